@@ -201,7 +201,9 @@ int pepsmg_vv_dot_device_noalloc(int32_t nx, int32_t ny, int32_t nz, const doubl
  * once, each output written once), *kernel_name the kernel's symbol (a
  * per-thread buffer, valid until the calling thread's next call).  As in a
  * solve, a launch that follows an upward one marches down (the symbol's
- * k_rb_fused_down twin), so the launches alternate between the two. */
+ * k_rb_fused_down twin), so the launches alternate between the two; on
+ * levels where the solver runs two iterations in a launch (k_sweep), so does
+ * this hook, and the time and bytes are those of such a launch. */
 int pepsmg_bench_smoother(pepsmg_ctx *ctx, int32_t precision, int32_t reps, double omega,
                           double *avg_ms, double *bytes, const char **kernel_name);
 
@@ -209,7 +211,8 @@ int pepsmg_bench_smoother(pepsmg_ctx *ctx, int32_t precision, int32_t reps, doub
  * following solve on ctx bracket the plain red/black smoother launches on its
  * finest level (FP64; in precision 1 the FP32 smoother) with HIP events on
  * the solve stream, and clears the totals; 0 stops.  Up to 256 launches per
- * solve are timed, both upward and downward ones (k_rb_fused_down). */
+ * solve are timed, both upward and downward ones (k_rb_fused_down); where
+ * the finest level's plain launches are two iterations each (k_sweep), those. */
 int pepsmg_kernel_timing(pepsmg_ctx *ctx, int32_t enable);
 
 /* Totals since the last pepsmg_kernel_timing(ctx, 1) (kept when timing is

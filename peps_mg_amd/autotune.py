@@ -76,6 +76,11 @@ def tune_tiles(sdm, nlevel, precision, reps=10, use_cache=True):
         _lib.check(_lib.lib().pepsmg_bench_smoother(mg.h, precision, reps, 1.0, C.byref(avg), C.byref(nb),
                                                     C.byref(kn)))
         timings[f"{tx}x{ty}/pf{pf}"] = avg.value
+        if kn.value.startswith(b"k_sweep"):
+            # this level's smoother takes two iterations a pass and has no tile to choose; the
+            # levels below keep the tile of their size
+            best_ms, best = avg.value, {"tile_x": 0, "tile_y": 0, "fused_smoother": 1}
+            break
         if avg.value < best_ms:
             best_ms, best = avg.value, {"tile_x": tx, "tile_y": ty, "fused_smoother": pf}
     mg.destroy()

@@ -233,6 +233,7 @@ static int upload_level(const HostLevel& h, DevLevel<T>& d, bool with_transfer) 
   d.px = pitch_for(d.nx);
   d.pxy = d.px * d.ny;
   d.ncell = (size_t)d.pxy * d.nz;
+  d.find_zrun(h.cw[2], h.ce[2]);
   for (int a = 0; a < 3; a++) {
     d.cw[a] = dupload(conv<double, T>(h.cw[a]), &rc);
     d.ce[a] = dupload(conv<double, T>(h.ce[a]), &rc);

@@ -64,6 +64,20 @@ struct DevLevel {
   T *rw[3] = {nullptr, nullptr, nullptr}, *pp[3] = {nullptr, nullptr, nullptr}, *pn[3] = {nullptr, nullptr, nullptr};
   int rs[3] = {1, 1, 1}, ps[3] = {1, 1, 1};
   T *x = nullptr, *b = nullptr, *r = nullptr, *x2 = nullptr;
+  // longest run of planes zlo .. zhi with the same z coefficients (c5u, c6u)
+  int zlo = 1, zhi = 0;
+  T c5u = T(0), c6u = T(0);
+  void find_zrun(const std::vector<double>& cwz, const std::vector<double>& cez) {
+    for (int k = 1, start = 1; k <= nz; k++) {
+      if ((T)cwz[k] != (T)cwz[start] || (T)cez[k] != (T)cez[start]) start = k;
+      if (k - start > zhi - zlo) {
+        zlo = start;
+        zhi = k;
+        c5u = (T)cwz[k];
+        c6u = (T)cez[k];
+      }
+    }
+  }
   bool fused_up = false;                  // the last fused smoother launch on this level marched up
 
   Lvl<T> L() const {

@@ -15,6 +15,7 @@
 #include "pepsmg_fused.h"
 #include "pepsmg_internal.h"
 #include "pepsmg_march.h"
+#include "pepsmg_sweep.h"
 
 namespace pepsmg {
 
@@ -257,7 +258,7 @@ struct Ops {
     int ty = ty_used(d);
     const bool down = next_down(d, mode);
     bool timed;
-    timer_begin(d, mode, timed);
+    timer_begin(d, timer && sweeps(d) ? 1 : mode, timed);   // (where k_sweep is the plain kernel, it alone is timed)
     if (sizeof(T) == 4 && tx_used(d) == 64) fused_tx<64>(d, omega, mode, ty, partial, down);
     else fused_tx<FTX>(d, omega, mode, ty, partial, down);
     timer_end(timed);
@@ -269,14 +270,154 @@ struct Ops {
     int ty = ty_used(d);
     const bool down = next_down(d, 0);
     bool timed;
-    timer_begin(d, 0, timed);
+    timer_begin(d, timer && sweeps(d) ? 1 : 0, timed);
     if (sizeof(T) == 4 && tx_used(d) == 64) fused_tx<64>(d, omega, 0, ty, nullptr, down);
     else fused_tx<FTX>(d, omega, 0, ty, nullptr, down);
     timer_end(timed);
     fused_out = nullptr;
   }
-  // symbol of the plain fused kernel fused_iter launches on level d
-  void fused_name(const DevLevel<T>& d, char* buf, size_t n) const {
+  // Tiles of one axis: the fewest that cover n cells when a tile holds `span`
+  // cells, ring included (none at the domain's faces); the cells each
+  // stores come out even, the first of every tile odd.
+  static void sweep_axis(int n, int span, int ring, int& tiles, int& use) {
+    auto even = [](int v) { return (v + 1) / 2 * 2; };
+    if (n <= span) {
+      tiles = 1;
+      use = even(n);
+      return;
+    }
+    tiles = 2;
+    while (even((n + tiles - 1) / tiles) > span - (tiles > 2 ? 2 * ring : ring)) tiles++;
+    use = even((n + tiles - 1) / tiles);
+    tiles = (n + use - 1) / use;
+  }
+
+  static int cu_count() {
+    static std::mutex mu;
+    static std::map<int, int> cache;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 256;
+    std::lock_guard<std::mutex> lock(mu);
+    auto it = cache.find(dev);
+    if (it != cache.end()) return it->second;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
+    return cache[dev] = cus;
+  }
+
+  // One block of the sweep kernels runs per CU.  A chunk of kc planes takes
+  // kc + 2 ring + 1 plane steps, in groups of NS; of the chunk sizes with the
+  // fewest groups over all waves of blocks the smallest is taken (more than
+  // four waves of blocks never pay: every chunk adds its ring).
+  // *share: the level's cells over the cells of all block steps.
+  template <typename S>
+  static SweepGrid sweep_grid(const DevLevel<T>& d, double* share = nullptr) {
+    SweepGrid G;
+    sweep_axis(d.nx, SW_COLS, S::RINGX, G.gx, G.uw);
+    sweep_axis(d.ny, S::ROWS, S::RING, G.gy, G.uh);
+    const long tiles = (long)G.gx * G.gy, cus = cu_count();
+    long best = -1;
+    G.kchunk = 2;
+    for (long nch = 1; nch <= std::max(1L, 4 * cus / tiles); nch++) {
+      const long kc = (d.nz + 2 * nch - 1) / (2 * nch) * 2;
+      const long waves = (tiles * ((d.nz + kc - 1) / kc) + cus - 1) / cus;
+      const long cost = waves * ((kc + 2 * S::RING + S::NS) / S::NS);
+      if (best < 0 || cost <= best) {
+        best = cost;
+        G.kchunk = (int)kc;
+      }
+    }
+    G.nch = (d.nz + G.kchunk - 1) / G.kchunk;
+    if (share) *share = (double)d.cells() / ((double)best * S::NS * cus * SW_COLS * S::ROWS);
+    return G;
+  }
+
+  // Whether two iterations on level d run in one pass (k_sweep) rather than
+  // in two (k_rb_fused): from 4 M cells on, and where a fair share of the
+  // work is on cells of the level (thin levels leave the 128-column tiles or
+  // the chunks mostly ring).  Solves, both ways:
+  // FP64 128^3 (share 0.11) 3.29 against 3.13 ms, 160^3 (0.16) 4.99 against
+  // 5.10, 192^3 5.08 against 5.35, 320^3 13.5 against 15.4, 512^3 39.1
+  // against 42.8; mixed 128^3 (0.11) 1.55 against 1.57, 160^3 1.97 against 2.21, 256^3 3.22 against 3.78, 384^3 6.49
+  // against 9.89, 512^3 13.1 against 17.5.  (A plane's row offsets are
+  // 32-bit bytes.)
+  static bool sweeps(const DevLevel<T>& d) {
+    if (d.cells() < 4000000L || d.pxy * (long)sizeof(T) > 0x7fffffffL) return false;
+    double share = 0.0;
+    sweep_grid<SweepShape<T, SW_WAVES, 2, SW_X>>(d, &share);
+    return share >= 0.15;
+  }
+
+  // NIT red/black iterations on level d in one pass, x -> x2, then swap.
+  // PRE: from x, from 0, or from x + P x_c (c the next coarser level, every
+  // axis halving).  to_caller (FP64): the caller's solution also receives x.
+  template <int NIT, int PRE>
+  void sweep(DevLevel<T>& d, const DevLevel<T>* c, T omega, bool to_caller = false) {
+    using S = SweepShape<T, SW_WAVES, NIT, PRE>;
+    SweepArgs<T> A;
+    std::memset(&A, 0, sizeof A);
+    A.xo = d.x2;
+    A.xi = d.x;
+    A.b = d.b;
+    A.L = d.L();
+    A.omega = omega;
+    A.zlo = d.zlo;
+    A.zhi = d.zhi;
+    A.c5u = d.c5u;
+    A.c6u = d.c6u;
+    if (PRE == SW_PROLONG) {
+      A.xc = c->x;
+      A.C = c->L();
+      A.W = d.PW();
+    }
+    if (to_caller) {
+      A.ext = caller_sol;
+      A.U = caller_lvl;
+    }
+    A.G = sweep_grid<S>(d);
+    const unsigned nb = (unsigned)((A.G.gx * A.G.gy * A.G.nch + 7) / 8 * 8);
+    bool timed;
+    timer_begin(d, PRE == SW_X && !to_caller ? 0 : 1, timed);
+    set_dynamic_lds((const void*)k_sweep<T, SW_WAVES, NIT, PRE>, S::LDS * sizeof(T));   // a failure surfaces at the solve's end
+    hipLaunchKernelGGL((k_sweep<T, SW_WAVES, NIT, PRE>), dim3(nb), dim3(S::THREADS), S::LDS * sizeof(T), s, A);
+    timer_end(timed);
+    d.fused_up = true;
+    std::swap(d.x, d.x2);
+  }
+
+  // nu red/black iterations on level d (x -> x): by twos where that is the
+  // faster way, one by one otherwise.  zero_start: from x = 0; c: from
+  // x + P x_c; last_mode: fused-kernel mode of the last iteration (4: it also
+  // stores x into the caller's array).
+  void iterate(DevLevel<T>& d, T omega, int nu, bool zero_start = false, DevLevel<T>* c = nullptr,
+               int last_mode = 0) {
+    const bool two = nu >= 2 && sweeps(d);
+    int it = 0;
+    if (c) {
+      // FP64 keeps the separate prolongation: with the coarse planes beside
+      // the fine ones the kernel needs more than the 256 registers there are
+      bool done = false;
+      if constexpr (sizeof(T) == 4) {
+        if (two && d.ps[0] == 2 && d.ps[1] == 2 && d.ps[2] == 2) {
+          sweep<2, SW_PROLONG>(d, c, omega);
+          it = 2;
+          done = true;
+        }
+      }
+      if (!done) prolong_add(d, *c, d.x);
+    } else if (zero_start && two) {
+      sweep<2, SW_ZERO>(d, nullptr, omega);
+      it = 2;
+    }
+    for (; two && it + 2 <= nu; it += 2) sweep<2, SW_X>(d, nullptr, omega, it + 2 == nu && last_mode == 4);
+    for (; it < nu; it++) fused_iter(d, omega, (it == 0 && zero_start) ? 1 : (it == nu - 1 && last_mode ? last_mode : 0));
+  }
+
+  // symbol of the plain smoother kernel iterate launches on level d
+  void smoother_name(const DevLevel<T>& d, char* buf, size_t n) const {
+    if (sweeps(d)) {
+      std::snprintf(buf, n, "k_sweep<%s, %d, 2, 0>", sizeof(T) == 8 ? "double" : "float", SW_WAVES);
+      return;
+    }
     const int ty = ty_used(d);
     std::snprintf(buf, n, "k_rb_fused<%s, %d, %d, 0, %d>", sizeof(T) == 8 ? "double" : "float", tx_used(d), ty,
                   ty == 32 ? 1 : prefetch);   // 32-row tiles load one plane ahead

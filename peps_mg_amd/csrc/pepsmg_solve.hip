@@ -251,7 +251,7 @@ static void timer_attach(pepsmg_ctx* c, Ops<T>& op, DevLevel<T>& d) {
   op.timer = &c->timer;
   c->timer.level = &d;
   c->timer.used = 0;
-  op.fused_name(d, c->timer.name, sizeof c->timer.name);
+  op.smoother_name(d, c->timer.name, sizeof c->timer.name);
 }
 
 // Adds the bracketed launches of the finished solve to the totals.
@@ -279,18 +279,17 @@ static void smooth_level(pepsmg_ctx* c, Ops<T>& op, Hier<T>& h, CgBufs<T>* cg, i
                          bool zero_start, bool prolong_first, int last_mode = 0) {
   DevLevel<T>& d = h.lv[l];
   bool fused = c->opt.fused_smoother && c->opt.smoother == 0 && nu > 0;
+  if (fused) {
+    op.iterate(d, omega, nu, zero_start, prolong_first ? &h.lv[l + 1] : nullptr, last_mode);
+    return;
+  }
   if (prolong_first) op.prolong_add(d, h.lv[l + 1], d.x);
   if (c->opt.smoother == 1) {
     cg_iterate(op, d, d.x, d.b, d.r, cg->p[l], cg->p2[l], cg->ap[l], nu, zero_start, c->d_partial,
                c->d_scalars + 8);
     return;
   }
-  if (!fused) {
-    op.rbgs(d, d.x, d.b, nu, omega, zero_start);
-    return;
-  }
-  for (int it = 0; it < nu; it++)
-    op.fused_iter(d, omega, (it == 0 && zero_start) ? 1 : (it == nu - 1 && last_mode ? last_mode : 0));
+  op.rbgs(d, d.x, d.b, nu, omega, zero_start);
 }
 
 // Coarsest level: FP64 solve in one workgroup (src/multigrid.f90:1944-1949,
@@ -966,8 +965,9 @@ int pepsmg_bench_smoother(pepsmg_ctx* c, int32_t precision, int32_t reps, double
   float ms = 0;
   double n = 0;
   const bool fused = c->opt.fused_smoother != 0;
-  // fused: one red+black iteration reads x and b and writes x once (3 n
-  // elements); colour sweep: reads x and b, writes half of x (2 n)
+  // fused: a launch (two iterations where k_sweep is the solver's kernel,
+  // else one) reads x and b and writes x once (3 n elements); colour sweep:
+  // reads x and b, writes half of x (2 n)
   auto run = [&](auto& op, auto& d, const char* tname) -> int {
     op.tile_y = c->opt.tile_y;
     op.tile_x = c->opt.tile_x;
@@ -975,7 +975,8 @@ int pepsmg_bench_smoother(pepsmg_ctx* c, int32_t precision, int32_t reps, double
     using T = typename std::remove_reference<decltype(d.x[0])>::type;
     auto body = [&]() {
       for (int q = 0; q < reps; q++) {
-        if (fused) op.fused_iter(d, (T)omega, 0);
+        if (fused && op.sweeps(d)) op.template sweep<2, SW_X>(d, nullptr, (T)omega);
+        else if (fused) op.fused_iter(d, (T)omega, 0);
         else op.smooth_colour(d, d.b, d.x, (T)omega, q & 1, false);
       }
     };
@@ -985,8 +986,7 @@ int pepsmg_bench_smoother(pepsmg_ctx* c, int32_t precision, int32_t reps, double
     HIP_TRY(hipEventRecord(c->ev1, c->stream));
     n = (double)d.cells();
     if (fused)
-      std::snprintf(name, sizeof name, "k_rb_fused<%s, %d, %d, 0, %d>", tname, op.tx_used(d), op.ty_used(d),
-                    op.ty_used(d) == 32 ? 1 : op.prefetch);   // 32-row tiles load one plane ahead
+      op.smoother_name(d, name, sizeof name);
     else
       std::snprintf(name, sizeof name, "k_rb_colour<%s, false>", tname);
     return PEPSMG_OK;
@@ -1073,6 +1073,7 @@ struct OneLevelT {
     d.px = pitch_for(d.nx);
     d.pxy = d.px * d.ny;
     d.ncell = (size_t)d.pxy * d.nz;
+    d.find_zrun(h.cw[2], h.ce[2]);
     for (int a = 0; a < 3; a++) {
       const std::vector<T> cw(h.cw[a].begin(), h.cw[a].end()), ce(h.ce[a].begin(), h.ce[a].end());
       HIP_TRY(hipMalloc(&d.cw[a], cw.size() * sizeof(T)));
@@ -1171,7 +1172,7 @@ int pepsmg_rbgs_iterator(const pepsmg_grid* grid, double* sol, const double* coe
   if (!rc) rc = o.upload(o.d.b, rhs);
   if (rc) return rc;
   Ops<double> op{o.s};
-  for (int it = 0; it < maxiteration; it++) op.fused_iter(o.d, omega, 0);
+  op.iterate(o.d, omega, maxiteration);
   return o.download(sol, o.d.x, 0);
 }
 
@@ -1184,7 +1185,7 @@ int pepsmg_rbgs_iterator_fp32(const pepsmg_grid* grid, double* sol, const double
   if (!rc) rc = o.upload(o.d.b, rhs);
   if (rc) return rc;
   Ops<float> op{o.s};
-  for (int it = 0; it < maxiteration; it++) op.fused_iter(o.d, (float)omega, 0);
+  op.iterate(o.d, (float)omega, maxiteration);
   return o.download(sol, o.d.x, 0);
 }
 
