@@ -94,6 +94,25 @@ __device__ __forceinline__ T diag(T c1, T c2, T c3, T c4, T c5, T c6) {
   return -(c1 + c2 + c3 + c4 + c5 + c6);
 }
 
+// Quotients by a fixed divisor c (FP64): a / c rounded exactly as the
+// division, from y = 1 / c (rounded).  The first correction leaves the
+// quotient within an ulp of a / c, the second then rounds correctly
+// (P. Markstein, IBM J. Res. Dev. 34, 1990): five operations against the
+// eleven, one of them at a quarter of the rate, of a division.  Holds
+// while no term underflows or overflows: |c| in 2^[-300, 300] and a = 0 or
+// |a| in 2^[-600, 600]; the callers divide outside that range.
+__device__ __forceinline__ double kd_quotient(double a, double c, double y) {
+  double q = a * y;
+  q = __builtin_fma(__builtin_fma(-c, q, a), y, q);
+  return __builtin_fma(__builtin_fma(-c, q, a), y, q);
+}
+// 0 .. KD_SPAN iff |a| lies in 2^[-600, 600] (a = 0 does not: it divides)
+constexpr unsigned KD_LOW = (1023u - 600u) << 21, KD_SPAN = 1200u << 21;
+__device__ __forceinline__ unsigned kd_range(double a) { return ((unsigned)__double2hiint(a) << 1) - KD_LOW; }
+__device__ __forceinline__ bool kd_divisor(double c) {
+  return fabs(c) >= 0x1p-300 && fabs(c) <= 0x1p300;
+}
+
 // A x at (i,j,k): mv_mul order, c0 term first (src/poisson_matrix_operator.f90:150-156)
 template <typename T>
 __device__ __forceinline__ T apply_at(const T* __restrict__ x, const Lvl<T>& L, int i, int j, int k) {

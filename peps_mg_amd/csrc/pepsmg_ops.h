@@ -612,7 +612,9 @@ inline bool pc_build(int L, Hier<double>& h64, size_t lds_max, Hier<T>& h, int s
   lc.pxy = (long)cd.nx * cd.ny;
   A.lc = lc;
   size_t nc = (size_t)cd.cells();
-  A.xcoff = (int)(take(nc * 8) / 8);
+  // x slots of pc_coarsest_small / pc_coarsest_block
+  A.xslots = nc > 64 && nc <= (size_t)PC_THREADS;
+  A.xcoff = (int)(take((nc <= 64 ? (size_t)PC_SMALL_X : A.xslots ? 2 * (nc + 1) : nc) * 8) / 8);
   A.bcoff = (int)(take(nc * 8) / 8);
   A.xctoff = (int)(take(nc * sizeof(T)) / sizeof(T));
   A.ccoff = (int)(take((size_t)pc_stage_elems(cd.nx, cd.ny, cd.nz, false) * 8) / 8);

@@ -295,6 +295,11 @@ static void smooth_level(pepsmg_ctx* c, Ops<T>& op, Hier<T>& h, CgBufs<T>* cg, i
 // Coarsest level: FP64 solve in one workgroup (src/multigrid.f90:1944-1949,
 // tolerance = the V-cycle tolerance, at most 1000 iterations).
 static void coarse_solve64(pepsmg_ctx* c, DevLevel<double>& d, double omega, double tol, int* slot) {
+  if (d.cells() > 1 && d.cells() <= 64) {
+    hipLaunchKernelGGL(k_coarse_small, dim3(1), dim3(COARSE_THREADS), 0, c->stream, d.x, d.b, d.L(), omega, tol, 1000,
+                       slot);
+    return;
+  }
   hipLaunchKernelGGL((k_coarse_solve<double>), dim3(1), dim3(COARSE_THREADS), 0, c->stream, d.x, d.b, d.L(),
                      omega, tol, 1000, (int*)nullptr, slot);
 }

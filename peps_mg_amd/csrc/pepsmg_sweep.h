@@ -87,25 +87,6 @@ __device__ __forceinline__ T sw_west(T v) { return sw_shift<0x138>(v); }   // wa
 template <typename T>
 __device__ __forceinline__ T sw_east(T v) { return sw_shift<0x130>(v); }   // wave_shl:1
 
-// Quotients by a fixed divisor c (FP64): a / c rounded exactly as the
-// division, from y = 1 / c (rounded).  The first correction leaves the
-// quotient within an ulp of a / c, the second then rounds correctly
-// (P. Markstein, IBM J. Res. Dev. 34, 1990): five operations against the
-// eleven, one of them at a quarter of the rate, of a division.  Holds
-// while no term underflows or overflows: |c| in 2^[-300, 300] and a = 0 or
-// |a| in 2^[-600, 600]; the callers divide outside that range.
-__device__ __forceinline__ double sw_quotient(double a, double c, double y) {
-  double q = a * y;
-  q = __builtin_fma(__builtin_fma(-c, q, a), y, q);
-  return __builtin_fma(__builtin_fma(-c, q, a), y, q);
-}
-// 0 .. SW_SPAN iff |a| lies in 2^[-600, 600] (a = 0 does not: it divides)
-constexpr unsigned SW_LOW = (1023u - 600u) << 21, SW_SPAN = 1200u << 21;
-__device__ __forceinline__ unsigned sw_range(double a) { return ((unsigned)__double2hiint(a) << 1) - SW_LOW; }
-__device__ __forceinline__ bool sw_divisor(double c) {
-  return fabs(c) >= 0x1p-300 && fabs(c) <= 0x1p300;
-}
-
 // A plane's address as one scalar in the global address space: the accesses
 // of its rows add a 32-bit lane offset to it (without this the compiler
 // keeps a 64-bit address per array and row in vector registers).
@@ -217,7 +198,7 @@ __global__ void __launch_bounds__(64 * W) k_sweep(SweepArgs<T> A) {
       if constexpr (F64) {
         dv[r][c] = c0;
         rv[r][c] = in ? 1.0 / c0 : 0.0;
-        kept = kept && (!in || sw_divisor(c0));
+        kept = kept && (!in || kd_divisor(c0));
       } else {
         rv[r][c] = in ? A.omega / c0 : T(0);
       }
@@ -475,10 +456,10 @@ __global__ void __launch_bounds__(64 * W) k_sweep(SweepArgs<T> A) {
 #pragma unroll
           for (int r = 0; r < R; r++) {
             a[r] = A.omega * diff(r, A.c5u, A.c6u);
-            far = max(far, sw_range(a[r]));
-            q[r] = sw_quotient(a[r], dv[r][cell(r)], rv[r][cell(r)]);
+            far = max(far, kd_range(a[r]));
+            q[r] = kd_quotient(a[r], dv[r][cell(r)], rv[r][cell(r)]);
           }
-          if (__builtin_amdgcn_ballot_w64(far > SW_SPAN)) {
+          if (__builtin_amdgcn_ballot_w64(far > KD_SPAN)) {
 #pragma unroll
             for (int r = 0; r < R; r++) q[r] = sw_fresh_v(rv[r][cell(r)]) != T(0) ? a[r] / dv[r][cell(r)] : T(0);
           }
