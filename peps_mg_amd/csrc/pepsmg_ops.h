@@ -598,7 +598,7 @@ inline bool pc_build(int L, Hier<double>& h64, size_t lds_max, Hier<T>& h, int s
     A.lv[q] = l;
     if (q < nlev - 1) {
       size_t n = (size_t)d.cells();
-      A.xoff[q] = (int)(take(n * sizeof(T)) / sizeof(T));
+      A.xoff[q] = (int)(take((n + 2) * sizeof(T)) / sizeof(T));   // two zeros behind it (pc_smooth_pairs)
       A.boff[q] = (int)(take(n * sizeof(T)) / sizeof(T));
       A.coff[q] = (int)(take((size_t)pc_stage_elems(d.nx, d.ny, d.nz, true) * sizeof(T)) / sizeof(T));
       A.rw[q] = d.RW();
