@@ -212,7 +212,9 @@ int pepsmg_bench_smoother(pepsmg_ctx *ctx, int32_t precision, int32_t reps, doub
  * finest level (FP64; in precision 1 the FP32 smoother) with HIP events on
  * the solve stream, and clears the totals; 0 stops.  Up to 256 launches per
  * solve are timed, both upward and downward ones (k_rb_fused_down); where
- * the finest level's plain launches are two iterations each (k_sweep), those. */
+ * the finest level's plain launches are two iterations each (k_sweep), those;
+ * on levels smoothed by blocks (k_block) every launch, counted with its
+ * iterations. */
 int pepsmg_kernel_timing(pepsmg_ctx *ctx, int32_t enable);
 
 /* Totals since the last pepsmg_kernel_timing(ctx, 1) (kept when timing is

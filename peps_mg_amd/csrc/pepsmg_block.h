@@ -1,0 +1,247 @@
+// pepsmg_block.h -- NIT red/black iterations on small levels in one launch
+// (gfx950): from x, from x = 0 or from x plus the prolongation of the coarser
+// level, out of place.
+//
+// Bound: latency.  On levels of 128^3 cells and fewer a z-march waits for a
+// memory round trip at each of its few plane steps (k_rb_fused takes 6 to 8
+// us on levels of 16^3 to 64^3, 3 of it such waits), and every iteration and
+// the prolongation is a launch of its own.  Here a block holds a BX x BY x BZ
+// tile and a ring of 2 NIT cells in LDS: all loads are issued at the start
+// (one round trip), the half-sweeps follow with a barrier each, every one on
+// a region one cell smaller, and the tile is stored.  Levels this small are
+// served from the caches, so the ring (7.5 times the tile's cells for 16 x 8
+// x 4 and two iterations) costs little beside the launches it saves.
+//
+// Threads own pairs (i odd, i + 1) of the region through the whole launch;
+// LDS keeps the first and the second cells of the pairs apart, so lanes touch
+// consecutive words.  Values, expressions and operand order are those of the
+// separate kernels (FP64 bit for bit).
+#pragma once
+#include "pepsmg_coarse.h"
+#include "pepsmg_sweep.h"
+
+namespace pepsmg {
+
+template <typename T>
+struct BlockArgs {
+  T* xo;
+  const T* xi;
+  const T* b;
+  const T* xc;               // SW_PROLONG: the coarser level's x
+  Lvl<T> L, C;
+  ProlongW<T> W;
+  T omega;
+  int gx, gy;                // tiles along x and y
+  double* partial;           // NORM: per-block sums of (b - A x_in)^2
+  T* ext;                    // FP64: the caller's array that also receives x_out (layout U), or null
+  Lvl<T> U;
+};
+
+template <int BX_, int BY_, int BZ_, int NT_>
+struct BlockTile {
+  static constexpr int BX = BX_, BY = BY_, BZ = BZ_, NT = NT_;
+};
+using BlockSmall = BlockTile<16, 8, 4, 512>;
+using BlockLarge = BlockTile<32, 8, 8, 1024>;
+
+template <typename T, typename B, int NIT, int PRE>
+struct BlockShape {
+  static constexpr int H = 2 * NIT;
+  static constexpr int PX = (B::BX + 2 * H) / 2, RY = B::BY + 2 * H, RZ = B::BZ + 2 * H;
+  static constexpr int NPAIR = PX * RY * RZ, PP = (NPAIR + B::NT - 1) / B::NT;
+  // coarse cells the region interpolates from
+  static constexpr int CX = PX + 2, CY = RY / 2 + 2, CZ = RZ / 2 + 2, NC = CX * CY * CZ;
+  static constexpr int PC = (NC + B::NT - 1) / B::NT;
+  static constexpr int LDS = 2 * NPAIR + 2 * (2 * PX + RY + RZ) + (PRE == SW_PROLONG ? NC : 0);   // elements
+};
+
+template <typename T, typename B, int NIT, int PRE, bool NORM>
+__global__ void __launch_bounds__(B::NT) k_block(BlockArgs<T> A) {
+  using S = BlockShape<T, B, NIT, PRE>;
+  using V2 = typename SwPair<T>::type;
+  constexpr bool F64 = sizeof(T) == 8;
+  constexpr int H = S::H, PX = S::PX, RY = S::RY, RZ = S::RZ, NP = S::NPAIR, PP = S::PP, NT = B::NT;
+  extern __shared__ __align__(16) unsigned char bl_smem[];
+  T* const xs = reinterpret_cast<T*>(bl_smem);       // first cells of the pairs, then the second ones
+  T* const cx = xs + 2 * NP;                         // cwx, cex of the region's columns (0 outside the level)
+  T* const cy = cx + 4 * PX;                         // cwy, cey of its rows
+  T* const cz = cy + 2 * RY;                         // cwz, cez of its planes
+  T* const cs = cz + 2 * RZ;                         // coarse cells
+
+  const Lvl<T>& L = A.L;
+  const int t = threadIdx.x;
+  const int bx = blockIdx.x % A.gx, byz = blockIdx.x / A.gx;
+  const int i0 = 1 + bx * B::BX - H, j0 = 1 + (byz % A.gy) * B::BY - H, k0 = 1 + (byz / A.gy) * B::BZ - H;   // i0 odd
+
+  // ---- all loads ----
+  V2 xv[PP], bv[PP];
+  int id[PP], dist[PP][2], at[PP];                   // at: pair, row and plane in the region
+  bool tile[PP], first[PP];                          // first: the pair's first cell is red (i + j + k odd)
+#pragma unroll
+  for (int p = 0; p < PP; p++) {
+    const int e = min(t + p * NT, NP - 1);
+    const int row = e / PX, px = e - row * PX, rz = row / RY, ry = row - rz * RY;
+    const int i = i0 + 2 * px, j = j0 + ry, k = k0 + rz;
+    const bool on = t + p * NT < NP;
+    const bool vr = on && j >= 1 && j <= L.ny && k >= 1 && k <= L.nz;
+    const bool v0 = vr && i >= 1 && i <= L.nx, v1 = vr && i + 1 >= 1 && i + 1 <= L.nx;
+    id[p] = e;
+    at[p] = px | ry << 8 | rz << 16;
+    // distance to the region's face (-1: outside the level), which half-sweeps count down
+    const int dyz = min(min(ry, RY - 1 - ry), min(rz, RZ - 1 - rz));
+    dist[p][0] = v0 ? min(dyz, min(2 * px, 2 * PX - 1 - 2 * px)) : -1;
+    dist[p][1] = v1 ? min(dyz, min(2 * px + 1, 2 * PX - 2 - 2 * px)) : -1;
+    first[p] = ((j + k) & 1) == 0;
+    tile[p] = v0 && px >= H / 2 && px < PX - H / 2 && ry >= H && ry < RY - H && rz >= H && rz < RZ - H;
+    // an odd column <= nx keeps the pair inside the padded row
+    const int ic = v0 ? i : 1, jc = min(max(j, 1), L.ny), kc = min(max(k, 1), L.nz);
+    const long g = lidx(L, ic, jc, kc);
+    if (PRE != SW_ZERO) xv[p] = *reinterpret_cast<const V2*>(A.xi + g);
+    bv[p] = *reinterpret_cast<const V2*>(A.b + g);
+  }
+  if (t < 2 * PX + RY + RZ) {
+    const int q = t - 2 * PX;
+    T w, e;
+    if (q < 0) {
+      const int i = i0 + t;
+      const bool in = i >= 1 && i <= L.nx;
+      w = in ? L.cwx[in ? i : 1] : T(0);
+      e = in ? L.cex[in ? i : 1] : T(0);
+    } else if (q < RY) {
+      const int j = min(max(j0 + q, 1), L.ny);
+      w = L.cwy[j];
+      e = L.cey[j];
+    } else {
+      const int k = min(max(k0 + q - RY, 1), L.nz);
+      w = L.cwz[k];
+      e = L.cez[k];
+    }
+    cx[2 * t] = w;
+    cx[2 * t + 1] = e;
+  }
+  if constexpr (PRE == SW_PROLONG) {
+    // coarse region: the parents of the fine region and one cell around
+    // (i0, j0 and k0 are odd: exact divisions)
+    const int ci = (i0 + 1) / 2 - 1, cj0 = (j0 + 1) / 2 - 1, ck0 = (k0 + 1) / 2 - 1;
+    T v[S::PC];
+#pragma unroll
+    for (int q = 0; q < S::PC; q++) {
+      const int e = min(t + q * NT, S::NC - 1);
+      const int row = e / S::CX, x = e - row * S::CX, z = row / S::CY, y = row - z * S::CY;
+      const int ic = ci + x, jc = cj0 + y, kc = ck0 + z;
+      const bool in = ic >= 1 && ic <= A.C.nx && jc >= 1 && jc <= A.C.ny && kc >= 1 && kc <= A.C.nz;
+      const T u = A.xc[lidx(A.C, min(max(ic, 1), A.C.nx), min(max(jc, 1), A.C.ny), min(max(kc, 1), A.C.nz))];
+      v[q] = in ? u : T(0);
+    }
+#pragma unroll
+    for (int q = 0; q < S::PC; q++)
+      if (t + q * NT < S::NC) cs[t + q * NT] = v[q];
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < PP; p++) {
+      const int px = at[p] & 255, ry = at[p] >> 8 & 255, rz = at[p] >> 16;
+      const int i = i0 + 2 * px, j = j0 + ry, k = k0 + rz;
+      if (dist[p][0] < 0) continue;                  // a halving level: both cells of a pair are in or out
+      const bool jo = j & 1, ko = k & 1;
+      const T sy = jo ? A.W.py_[j] : A.W.ny_[j], ny = jo ? A.W.py_[j + 1] : A.W.ny_[j - 1];
+      const T sz = ko ? A.W.pz_[k] : A.W.nz_[k], nz = ko ? A.W.pz_[k + 1] : A.W.nz_[k - 1];
+      const int jc = (j + 1) / 2 - cj0, kc = (k + 1) / 2 - ck0;
+      const T* P = cs + (kc * S::CY + jc) * S::CX + px + 1;        // the parent's row, at the pair's column
+      const int dy = jo ? -S::CX : S::CX, dz = (ko ? -S::CY : S::CY) * S::CX;
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        const T sx = c ? A.W.nx_[i + 1] : A.W.px_[i], nx = c ? A.W.nx_[i] : A.W.px_[i + 1];
+        const int dx = c ? 1 : -1;
+        const T num = sx * sy * sz * P[0] + nx * sy * sz * P[dx] + sx * ny * sz * P[dy] + sx * sy * nz * P[dz] +
+                      nx * ny * sz * P[dx + dy] + nx * sy * nz * P[dx + dz] + sx * ny * nz * P[dy + dz] +
+                      nx * ny * nz * P[dx + dy + dz];
+        const T add = num / ((sx + nx) * (sy + ny) * (sz + nz));
+        if (c) xv[p].y = xv[p].y + add;
+        else xv[p].x = xv[p].x + add;
+      }
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < PP; p++) {
+    if (t + p * NT < NP) {
+      xs[id[p]] = PRE != SW_ZERO && dist[p][0] >= 0 ? xv[p].x : T(0);
+      xs[NP + id[p]] = PRE != SW_ZERO && dist[p][1] >= 0 ? xv[p].y : T(0);
+    }
+  }
+  __syncthreads();
+
+  // neighbours of cell c of pair p: own array at +- a row or plane, the other
+  // array at the pair and beside it
+  auto temp = [&](int p, int c, T a1, T a2, T c3, T c4, T c5, T c6) -> T {
+    const T* o = xs + c * NP + id[p];
+    const T* w = xs + (1 - c) * NP + id[p] - (1 - c);
+    if constexpr (F64) return a1 * w[0] + a2 * w[1] + c3 * o[-PX] + c4 * o[PX] + c5 * o[-PX * RY] + c6 * o[PX * RY];
+    T d = a1 * w[0];
+    d = sw_fma(a2, w[1], d);
+    d = sw_fma(c3, o[-PX], d);
+    d = sw_fma(c4, o[PX], d);
+    d = sw_fma(c5, o[-PX * RY], d);
+    return sw_fma(c6, o[PX * RY], d);
+  };
+  if constexpr (NORM) {
+    double acc = 0.0;
+#pragma unroll
+    for (int p = 0; p < PP; p++) {
+      if (!tile[p]) continue;
+      const T *ky = cy + 2 * (at[p] >> 8 & 255), *kz = cz + 2 * (at[p] >> 16);
+      const T c3 = ky[0], c4 = ky[1], c5 = kz[0], c6 = kz[1];
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        if (dist[p][c] < 0) continue;
+        const T* kx = cx + 2 * (2 * (at[p] & 255) + c);
+        const T c0 = diag(kx[0], kx[1], c3, c4, c5, c6);
+        const T* o = xs + c * NP + id[p];
+        const T* w = xs + (1 - c) * NP + id[p] - (1 - c);
+        const T ax = c0 * o[0] + kx[0] * w[0] + kx[1] * w[1] + c3 * o[-PX] + c4 * o[PX] + c5 * o[-PX * RY] +
+                     c6 * o[PX * RY];
+        const T r = (c ? bv[p].y : bv[p].x) - ax;
+        acc += (double)r * (double)r;
+      }
+    }
+    __shared__ double sh[NT / 64];
+    const double s = block_sum(acc, sh);             // (its barriers also close the reads of x_in)
+    if (t == 0) A.partial[blockIdx.x] = s;
+  }
+#pragma unroll
+  for (int s = 1; s <= 2 * NIT; s++) {
+#pragma unroll
+    for (int p = 0; p < PP; p++) {
+      const bool c = first[p] == ((s & 1) == 0);     // the cell of this colour is the pair's second
+      if ((c ? dist[p][1] : dist[p][0]) < s) continue;
+      const T *ky = cy + 2 * (at[p] >> 8 & 255), *kz = cz + 2 * (at[p] >> 16);
+      const T c3 = ky[0], c4 = ky[1], c5 = kz[0], c6 = kz[1];
+      const T* kx = cx + 2 * (2 * (at[p] & 255) + c);
+      const T a1 = kx[0], a2 = kx[1], bb = c ? bv[p].y : bv[p].x;
+      T* o = xs + (c ? NP : 0) + id[p];
+      const T tm = PRE == SW_ZERO && s == 1 ? T(0) : temp(p, c, a1, a2, c3, c4, c5, c6);
+      const T xold = PRE == SW_ZERO && s == 1 ? T(0) : o[0];
+      if constexpr (F64) {
+        o[0] = sor_update(A.omega, bb, tm, diag(a1, a2, c3, c4, c5, c6), xold);
+      } else {
+        const T f = A.omega * __builtin_amdgcn_rcpf(a1 + a2 + (c3 + c4) + (c5 + c6));
+        o[0] = sw_fma(tm - bb, f, (T(1) - A.omega) * xold);
+      }
+    }
+    if (s < 2 * NIT) __syncthreads();
+  }
+  // the owner of a pair updated both of its cells last
+#pragma unroll
+  for (int p = 0; p < PP; p++) {
+    if (!tile[p]) continue;
+    const int i = i0 + 2 * (at[p] & 255), j = j0 + (at[p] >> 8 & 255), k = k0 + (at[p] >> 16);
+    const V2 o = {xs[id[p]], xs[NP + id[p]]};        // (a second cell beyond nx is 0 and lies in the row's padding)
+    *reinterpret_cast<V2*>(A.xo + lidx(L, i, j, k)) = o;
+    if (F64 && A.ext) {
+      T* u = A.ext + lidx(A.U, i, j, k);
+      if (dist[p][1] >= 0) st_pair_unal(u, o.x, o.y);
+      else u[0] = o.x;
+    }
+  }
+}
+
+}  // namespace pepsmg

@@ -15,7 +15,7 @@
 #include "pepsmg_fused.h"
 #include "pepsmg_internal.h"
 #include "pepsmg_march.h"
-#include "pepsmg_sweep.h"
+#include "pepsmg_block.h"
 
 namespace pepsmg {
 
@@ -240,9 +240,10 @@ struct Ops {
     timed = timer && timer->wants(&d, mode);
     if (timed) hipEventRecord(timer->ev[timer->used], s);
   }
-  void timer_end(bool timed) {
+  void timer_end(bool timed, int count = 1) {
     if (!timed) return;
     hipEventRecord(timer->ev[timer->used + 1], s);
+    timer->count[timer->used / 2] = count;
     timer->used += 2;
   }
   // A plain iteration that follows an upward launch on the same level
@@ -258,7 +259,7 @@ struct Ops {
     int ty = ty_used(d);
     const bool down = next_down(d, mode);
     bool timed;
-    timer_begin(d, timer && sweeps(d) ? 1 : mode, timed);   // (where k_sweep is the plain kernel, it alone is timed)
+    timer_begin(d, timer && (blocks(d) || sweeps(d)) ? 1 : mode, timed);   // (where k_sweep is the plain kernel, it alone is timed)
     if (sizeof(T) == 4 && tx_used(d) == 64) fused_tx<64>(d, omega, mode, ty, partial, down);
     else fused_tx<FTX>(d, omega, mode, ty, partial, down);
     timer_end(timed);
@@ -270,7 +271,7 @@ struct Ops {
     int ty = ty_used(d);
     const bool down = next_down(d, 0);
     bool timed;
-    timer_begin(d, timer && sweeps(d) ? 1 : 0, timed);
+    timer_begin(d, timer && (blocks(d) || sweeps(d)) ? 1 : 0, timed);
     if (sizeof(T) == 4 && tx_used(d) == 64) fused_tx<64>(d, omega, 0, ty, nullptr, down);
     else fused_tx<FTX>(d, omega, 0, ty, nullptr, down);
     timer_end(timed);
@@ -384,12 +385,87 @@ struct Ops {
     std::swap(d.x, d.x2);
   }
 
+  // Whether iterations on level d run by blocks of the level in LDS (k_block):
+  // up to 1.2 M cells in FP64 and 3 M in FP32, where the launches they save
+  // outweigh the rings.  Solves against one launch per iteration: FP64 16^3
+  // 0.80 against 0.93 ms, 64^3 1.57 against 1.76, 96^3 2.14 against 2.44 (by
+  // blocks on its 128^3 level, 128^3 takes 2.99 against 2.81); mixed 32^3 0.59
+  // against 0.70 ms, 64^3 0.80 against 0.99, 96^3 1.05 against 1.31, 128^3
+  // 1.47 against 1.54.
+  static bool blocks(const DevLevel<T>& d) { return d.cells() <= (sizeof(T) == 8 ? 1200000L : 3000000L); }
+  // 32 x 8 x 8 blocks of 1024 threads from 150000 cells on: less ring per cell
+  // (96^3 FP64 2.14 against 2.38 ms); below, 16 x 8 x 4 keeps more CUs busy
+  // (64^3 FP64 1.56 against 1.69 ms when its fine level, too, takes them)
+  static bool large_block(const DevLevel<T>& d) { return d.cells() > (sizeof(T) == 8 ? 300000L : 150000L); }
+
+  // NIT iterations on level d by blocks, x -> x2, then swap (PRE, c,
+  // to_caller as for sweep).  NORM (FP64, from x): the blocks' partial sums of
+  // |b - A x_in|^2 go to partial; returns their number.
+  template <typename B, int NIT, int PRE, bool NORM = false>
+  int block_launch(DevLevel<T>& d, const DevLevel<T>* c, T omega, bool to_caller, double* partial, T* out) {
+    using S = BlockShape<T, B, NIT, PRE>;
+    BlockArgs<T> A;
+    std::memset(&A, 0, sizeof A);
+    A.xo = out ? out : d.x2;
+    A.xi = d.x;
+    A.b = d.b;
+    A.L = d.L();
+    A.omega = omega;
+    if (PRE == SW_PROLONG) {
+      A.xc = c->x;
+      A.C = c->L();
+      A.W = d.PW();
+    }
+    if (to_caller) {
+      A.ext = caller_sol;
+      A.U = caller_lvl;
+    }
+    A.partial = partial;
+    A.gx = (d.nx + B::BX - 1) / B::BX;
+    A.gy = (d.ny + B::BY - 1) / B::BY;
+    const int nb = A.gx * A.gy * ((d.nz + B::BZ - 1) / B::BZ);
+    bool timed;
+    timer_begin(d, 0, timed);
+    if (S::LDS * sizeof(T) > 65536) set_dynamic_lds((const void*)k_block<T, B, NIT, PRE, NORM>, S::LDS * sizeof(T));
+    hipLaunchKernelGGL((k_block<T, B, NIT, PRE, NORM>), dim3((unsigned)nb), dim3(B::NT), S::LDS * sizeof(T), s, A);
+    timer_end(timed, NIT);
+    d.fused_up = true;
+    if (!out) std::swap(d.x, d.x2);
+    return nb;
+  }
+  template <int NIT, int PRE, bool NORM = false>
+  int block(DevLevel<T>& d, const DevLevel<T>* c, T omega, bool to_caller = false, double* partial = nullptr,
+            T* out = nullptr) {
+    return large_block(d) ? block_launch<BlockLarge, NIT, PRE, NORM>(d, c, omega, to_caller, partial, out)
+                          : block_launch<BlockSmall, NIT, PRE, NORM>(d, c, omega, to_caller, partial, out);
+  }
+
+  // iterate on a level of blocks
+  void iterate_blocks(DevLevel<T>& d, T omega, int nu, bool zero_start, DevLevel<T>* c, int last_mode) {
+    int it = 0;
+    auto last = [&](int n) { return it + n == nu && last_mode == 4; };
+    if (c && !(d.ps[0] == 2 && d.ps[1] == 2 && d.ps[2] == 2)) {
+      prolong_add(d, *c, d.x);
+      c = nullptr;
+    }
+    if (c && nu >= 2) block<2, SW_PROLONG>(d, c, omega, last(2)), it = 2;
+    else if (c) block<1, SW_PROLONG>(d, c, omega, last(1)), it = 1;
+    else if (zero_start && nu >= 2) block<2, SW_ZERO>(d, nullptr, omega), it = 2;
+    else if (zero_start) block<1, SW_ZERO>(d, nullptr, omega), it = 1;
+    for (; it + 2 <= nu; it += 2) block<2, SW_X>(d, nullptr, omega, last(2));
+    if (it < nu) block<1, SW_X>(d, nullptr, omega, last(1));
+  }
+
   // nu red/black iterations on level d (x -> x): by twos where that is the
   // faster way, one by one otherwise.  zero_start: from x = 0; c: from
   // x + P x_c; last_mode: fused-kernel mode of the last iteration (4: it also
   // stores x into the caller's array).
   void iterate(DevLevel<T>& d, T omega, int nu, bool zero_start = false, DevLevel<T>* c = nullptr,
                int last_mode = 0) {
+    if (blocks(d) && nu > 0) {
+      iterate_blocks(d, omega, nu, zero_start, c, last_mode);
+      return;
+    }
     const bool two = nu >= 2 && sweeps(d);
     int it = 0;
     if (c) {
@@ -414,6 +490,10 @@ struct Ops {
 
   // symbol of the plain smoother kernel iterate launches on level d
   void smoother_name(const DevLevel<T>& d, char* buf, size_t n) const {
+    if (blocks(d)) {
+      std::snprintf(buf, n, "k_block<%s", sizeof(T) == 8 ? "double" : "float");
+      return;
+    }
     if (sweeps(d)) {
       std::snprintf(buf, n, "k_sweep<%s, %d, 2, 0>", sizeof(T) == 8 ? "double" : "float", SW_WAVES);
       return;

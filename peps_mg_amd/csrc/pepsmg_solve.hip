@@ -261,7 +261,7 @@ static void timer_collect(pepsmg_ctx* c) {
     float ms = 0.0f;
     if (hipEventElapsedTime(&ms, t.ev[q], t.ev[q + 1]) == hipSuccess) {
       t.total_ms += ms;
-      t.launches++;
+      t.launches += t.count[q / 2];
     }
   }
   t.used = 0;
@@ -537,28 +537,40 @@ static int solve_fp64(pepsmg_ctx* c, int nu, double tol, double omega, pepsmg_st
     return hist[n - 1] * (hist[n - 1] / hist[n - 2]) < tol;
   };
   for (int cyc = first; cyc <= c->ncycle; cyc++) {
+    bool restricted = false;   // level 1's right-hand side is formed already
     if (fold) {
-      // first pre-smoothing iteration, with |b - A x|^2 of the incoming x (in
-      // cycle 1 of a direct solve from the caller's arrays)
-      op.fused_iter(f, omega, (cyc == 1 && direct) ? 3 : 2, c->d_partial);
-      hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, c->stream, c->d_partial, nbn,
+      // first pre-smoothing iteration (or two: by blocks), with |b - A x|^2
+      // of the incoming x (in cycle 1 of a direct solve from the caller's arrays)
+      const bool blk = op.blocks(f) && !(cyc == 1 && direct);
+      int nbc = nbn, pre_done = 1;
+      if (blk && nu >= 2) {
+        nbc = op.block<2, SW_X, true>(f, nullptr, omega, false, c->d_partial);
+        pre_done = 2;
+      } else if (blk) {
+        nbc = op.block<1, SW_X, true>(f, nullptr, omega, false, c->d_partial);
+      } else {
+        op.fused_iter(f, omega, (cyc == 1 && direct) ? 3 : 2, c->d_partial);
+      }
+      hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, c->stream, c->d_partial, nbc,
                          c->d_scalars + (cyc == 1 ? 0 : 1));
-      int pre_done = 1;
       if (cyc > 1) {
         HIP_TRY(hipMemcpyAsync(c->h_scalars, c->d_scalars, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(hipEventRecord(c->ev_norm, c->stream));
         // While the host waits for the norm, the GPU runs the second
-        // iteration into the spare buffer f.r; the first iteration's input,
-        // the answer if the tolerance is met, stays in f.x2.  Skipped when
-        // the check is predicted to stop the solve.
-        const bool ahead = nu >= 2 && !likely_converged();
+        // iteration into the spare buffer f.r (or, when both iterations are
+        // done, the restriction); the first launch's input, the answer if the
+        // tolerance is met, stays in f.x2.  Skipped when the check is
+        // predicted to stop the solve.
+        const bool ahead = !blk && nu >= 2 && !likely_converged();
         if (ahead) op.fused_iter_into(f, omega, f.r);
+        restricted = blk && pre_done == nu && !likely_converged();
+        if (restricted) op.residual_restrict(f, h.lv[1], f.x, f.b);          // :1932-1933
         HIP_TRY(hipEventSynchronize(c->ev_norm));
         res0 = c->h_scalars[0];
         int stop = check(cyc - 1, c->h_scalars[1]);
         if (stop < 0) return stop;
         if (stop) {
-          std::swap(f.x, f.x2);   // the solution is the iteration's input
+          std::swap(f.x, f.x2);   // the solution is the first launch's input
           c->sol_out_done = dual_cycle == cyc - 1;
           break;
         }
@@ -571,7 +583,7 @@ static int solve_fp64(pepsmg_ctx* c, int nu, double tol, double omega, pepsmg_st
     } else {
       smooth_level(c, op, h, cg, 0, nu, omega, false, false);            // :1931
     }
-    op.residual_restrict(f, h.lv[1], f.x, f.b);                            // :1932-1933
+    if (!restricted) op.residual_restrict(f, h.lv[1], f.x, f.b);           // :1932-1933
     int* slot = (cyc - 1 < c->citers_cap) ? c->d_citers + (cyc - 1) : nullptr;
     vcycle_coarse_part<double>(c, op, h, cg, nu, nu, omega, tol, slot);    // :1936-1962
     const bool dual = ends_solve(cyc);
@@ -980,7 +992,8 @@ int pepsmg_bench_smoother(pepsmg_ctx* c, int32_t precision, int32_t reps, double
     using T = typename std::remove_reference<decltype(d.x[0])>::type;
     auto body = [&]() {
       for (int q = 0; q < reps; q++) {
-        if (fused && op.sweeps(d)) op.template sweep<2, SW_X>(d, nullptr, (T)omega);
+        if (fused && op.blocks(d)) op.template block<1, SW_X>(d, nullptr, (T)omega);
+        else if (fused && op.sweeps(d)) op.template sweep<2, SW_X>(d, nullptr, (T)omega);
         else if (fused) op.fused_iter(d, (T)omega, 0);
         else op.smooth_colour(d, d.b, d.x, (T)omega, q & 1, false);
       }
@@ -1019,6 +1032,7 @@ int pepsmg_kernel_timing(pepsmg_ctx* c, int32_t enable) {
   if (enable && t.ev.empty()) {
     constexpr int POOL = 512;   // 256 timed launches per solve
     t.ev.resize(POOL, nullptr);
+    t.count.resize(POOL / 2, 1);
     for (auto& e : t.ev) HIP_TRY(hipEventCreate(&e));
   }
   t.on = enable != 0;
