@@ -52,7 +52,8 @@ struct BlockShape {
   // coarse cells the region interpolates from
   static constexpr int CX = PX + 2, CY = RY / 2 + 2, CZ = RZ / 2 + 2, NC = CX * CY * CZ;
   static constexpr int PC = (NC + B::NT - 1) / B::NT;
-  static constexpr int LDS = 2 * NPAIR + 2 * (2 * PX + RY + RZ) + (PRE == SW_PROLONG ? NC : 0);   // elements
+  static constexpr int NW = 2 * (2 * PX + RY + RZ);        // coefficients (or weights) of the region's lines
+  static constexpr int LDS = 2 * NPAIR + NW + (PRE == SW_PROLONG ? NW + NC : 0);   // elements
 };
 
 template <typename T, typename B, int NIT, int PRE, bool NORM>
@@ -66,7 +67,8 @@ __global__ void __launch_bounds__(B::NT) k_block(BlockArgs<T> A) {
   T* const cx = xs + 2 * NP;                         // cwx, cex of the region's columns (0 outside the level)
   T* const cy = cx + 4 * PX;                         // cwy, cey of its rows
   T* const cz = cy + 2 * RY;                         // cwz, cez of its planes
-  T* const cs = cz + 2 * RZ;                         // coarse cells
+  T* const pw = cx + S::NW;                          // SW_PROLONG: weights of parent and neighbour, as cx, cy, cz
+  T* const cs = pw + S::NW;                          // SW_PROLONG: coarse cells
 
   const Lvl<T>& L = A.L;
   const int t = threadIdx.x;
@@ -118,6 +120,17 @@ __global__ void __launch_bounds__(B::NT) k_block(BlockArgs<T> A) {
     }
     cx[2 * t] = w;
     cx[2 * t + 1] = e;
+    if constexpr (PRE == SW_PROLONG) {
+      // odd cell: p(f), p(f + 1); even cell: n(f), n(f - 1)
+      const int axis = q < 0 ? 0 : q < RY ? 1 : 2;
+      const int f = axis == 0 ? i0 + t : axis == 1 ? j0 + q : k0 + q - RY;
+      const int n = axis == 0 ? L.nx : axis == 1 ? L.ny : L.nz;
+      const T* p = axis == 0 ? A.W.px_ : axis == 1 ? A.W.py_ : A.W.pz_;
+      const T* m = axis == 0 ? A.W.nx_ : axis == 1 ? A.W.ny_ : A.W.nz_;
+      const int g = min(max(f, 1), n);
+      pw[2 * t] = g & 1 ? p[g] : m[g];
+      pw[2 * t + 1] = g & 1 ? p[g + 1] : m[g - 1];
+    }
   }
   if constexpr (PRE == SW_PROLONG) {
     // coarse region: the parents of the fine region and one cell around
@@ -140,17 +153,17 @@ __global__ void __launch_bounds__(B::NT) k_block(BlockArgs<T> A) {
 #pragma unroll
     for (int p = 0; p < PP; p++) {
       const int px = at[p] & 255, ry = at[p] >> 8 & 255, rz = at[p] >> 16;
-      const int i = i0 + 2 * px, j = j0 + ry, k = k0 + rz;
+      const int j = j0 + ry, k = k0 + rz;
       if (dist[p][0] < 0) continue;                  // a halving level: both cells of a pair are in or out
       const bool jo = j & 1, ko = k & 1;
-      const T sy = jo ? A.W.py_[j] : A.W.ny_[j], ny = jo ? A.W.py_[j + 1] : A.W.ny_[j - 1];
-      const T sz = ko ? A.W.pz_[k] : A.W.nz_[k], nz = ko ? A.W.pz_[k + 1] : A.W.nz_[k - 1];
+      const T *wx = pw + 4 * px, *wy = pw + 4 * PX + 2 * ry, *wz = pw + 4 * PX + 2 * RY + 2 * rz;
+      const T sy = wy[0], ny = wy[1], sz = wz[0], nz = wz[1];
       const int jc = (j + 1) / 2 - cj0, kc = (k + 1) / 2 - ck0;
       const T* P = cs + (kc * S::CY + jc) * S::CX + px + 1;        // the parent's row, at the pair's column
       const int dy = jo ? -S::CX : S::CX, dz = (ko ? -S::CY : S::CY) * S::CX;
 #pragma unroll
       for (int c = 0; c < 2; c++) {
-        const T sx = c ? A.W.nx_[i + 1] : A.W.px_[i], nx = c ? A.W.nx_[i] : A.W.px_[i + 1];
+        const T sx = wx[2 * c], nx = wx[2 * c + 1];
         const int dx = c ? 1 : -1;
         const T num = sx * sy * sz * P[0] + nx * sy * sz * P[dx] + sx * ny * sz * P[dy] + sx * sy * nz * P[dz] +
                       nx * ny * sz * P[dx + dy] + nx * sy * nz * P[dx + dz] + sx * ny * nz * P[dy + dz] +

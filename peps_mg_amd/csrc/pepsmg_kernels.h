@@ -350,6 +350,43 @@ static __global__ void __launch_bounds__(RED_THREADS) k_dot_final(const double* 
   if (threadIdx.x == 0) *out = s;
 }
 
+// A scalar of the CG smoother as the partial sums it consists of: every block
+// of the kernel that needs it adds them up itself, in k_dot_final's order (so
+// all get k_dot_final's value), instead of waiting for a launch of one block
+// in between.  n = 1: the scalar itself.
+struct PartialSum {
+  const double* p;
+  int n;
+};
+// The quotient num / den of two such scalars on every thread; both sums are
+// formed side by side (sh: 2 RED_THREADS / 64 doubles).
+__device__ __forceinline__ double partial_ratio(const PartialSum& num, const PartialSum& den, double* sh) {
+  constexpr int NW = RED_THREADS / 64;
+  double a = 0.0, d = 0.0;
+  const int n = max(num.n, den.n);
+  for (int c = threadIdx.x; c < n; c += RED_THREADS) {
+    const double u = c < num.n ? num.p[c] : 0.0, v = c < den.n ? den.p[c] : 0.0;
+    if (c < num.n) a += u;
+    if (c < den.n) d += v;
+  }
+  for (int o = 32; o > 0; o >>= 1) {   // wave_sum
+    a += __shfl_down(a, o, 64);
+    d += __shfl_down(d, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    sh[threadIdx.x >> 6] = a;
+    sh[NW + (threadIdx.x >> 6)] = d;
+  }
+  __syncthreads();
+  double s = 0.0, t = 0.0;             // block_sum's sum over the waves, by every thread
+  for (int q = 0; q < NW; q++) {
+    s += sh[q];
+    t += sh[NW + q];
+  }
+  __syncthreads();
+  return s / t;
+}
+
 // ---------------------------------------------------------------------------
 // Coarsest-level solve in one workgroup (src/multigrid.f90:1819-1851 ->
 // rbgs_solver_poisson_matrix, src/rbgs_poisson_matrix.f90:47-179).  x is

