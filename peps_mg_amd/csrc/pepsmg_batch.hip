@@ -18,9 +18,10 @@
 // FP32 V-cycles inside FP64 iterative refinement (inner_cycles V-cycles per
 // refinement step).  A replay is one V-cycle (FP64) or one refinement step
 // (mixed); the host reads one counter of still-active items per replay.
-// The values an item gets are exactly those of its single-grid solve with
-// the same options (same kernels, same order), except that the final
-// refinement step always runs inner_cycles cycles.
+// In FP64 the values an item gets are exactly those of its single-grid solve
+// with the same options.  Mixed precision: which smoother kernel serves a
+// level follows the batch's cells, not the item's, and the FP32 kernels round
+// differently; the final refinement step always runs inner_cycles cycles.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -57,6 +58,18 @@ struct FusedItem {
   const T* b;
   Lvl<T> L;
   FusedGrid G;
+};
+
+template <typename T>
+struct SweepItem {
+  int block0, item;
+  SweepArgs<T> A;
+};
+
+template <typename T>
+struct BlockItem {
+  int block0, item;
+  BlockArgs<T> A;
 };
 
 template <typename T>
@@ -101,6 +114,26 @@ kb_rb_fused(const FusedItem<T>* __restrict__ items, int n, const int* __restrict
   if (!active[it.item]) return;
   rb_fused_block<T, TX, TY, MODE, PF>(blockIdx.x - it.block0, it.xo, it.xi, it.b, it.L, omega, it.G, nullptr, it.L,
                                       (T*)nullptr);
+}
+
+// nb: blocks of all items (the grid is rounded up to a multiple of 8)
+template <typename T, int NIT, int PRE>
+__global__ void __launch_bounds__(64 * SW_WAVES)
+kb_sweep(const SweepItem<T>* __restrict__ items, int n, int nb, const int* __restrict__ active) {
+  const int lin = sweep_block();
+  if (lin >= nb) return;
+  const int q = batch_find(items, n, lin);
+  if (!active[items[q].item]) return;
+  const SweepArgs<T> A = items[q].A;
+  sweep_tile<T, SW_WAVES, NIT, PRE>(A, lin - items[q].block0);
+}
+
+template <typename T, typename B, int NIT, int PRE>
+__global__ void __launch_bounds__(B::NT)
+kb_block(const BlockItem<T>* __restrict__ items, int n, const int* __restrict__ active) {
+  const int q = batch_find(items, n, blockIdx.x);
+  if (!active[items[q].item]) return;
+  block_tile<T, B, NIT, PRE, false>(items[q].A, blockIdx.x - items[q].block0);
 }
 
 template <typename T>
@@ -206,6 +239,7 @@ struct BItem {
 struct Sched {
   std::vector<char> host;
   std::vector<std::function<void(hipStream_t, const char*)>> ops;
+  hipError_t err = hipSuccess;   // a kernel's LDS request that was refused
   template <typename X>
   size_t put(const std::vector<X>& v) {
     size_t off = (host.size() + 255) / 256 * 256;
@@ -297,13 +331,11 @@ namespace pepsmg {
 // fine-level residual-march grid (same decomposition as the single-grid solver)
 static MarchGrid resid_grid(const DevLevel<double>& f) { return Ops<double>::march_grid(f, RESID_TY, false); }
 
-// Record nu fused iterations on level l of every item that has it (per-level
-// levels only), swapping each item's x / x2 as the launches do.  Items are
-// grouped by fused-smoother tile shape, one launch per group.  zero_first:
-// the first iteration starts from x = 0.
+// One red/black iteration on level l of the given items, swapping each item's
+// x / x2 as the launch does.  zero: from x = 0.
 template <typename T, int TX, int TY>
-static void rec_smooth_group(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, const std::vector<int>& members,
-                             int l, bool zero, T omega) {
+static void rec_fused(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, const std::vector<int>& members, int l,
+                      bool zero, T omega) {
   std::vector<FusedItem<T>> tab;
   int nb = 0;
   for (int i : members) {
@@ -331,31 +363,258 @@ static void rec_smooth_group(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H
   });
 }
 
+// Decompositions of one sweep launch over several levels; returns their cells
+// over the cells of all block steps.  One block runs per CU, so the levels
+// share a chunk size: that with the fewest groups of plane steps over all
+// waves of blocks.
+template <typename T, int NIT, int PRE>
+static double sweep_grids(const std::vector<const DevLevel<T>*>& lv, std::vector<SweepGrid>& grids) {
+  using S = SweepShape<T, SW_WAVES, NIT, PRE>;
+  const long cus = Ops<T>::cu_count();
+  grids.resize(lv.size());
+  int nz = 2;
+  double cells = 0.0;
+  for (size_t q = 0; q < lv.size(); q++) {
+    Ops<T>::sweep_axis(lv[q]->nx, SW_COLS, S::RINGX, grids[q].gx, grids[q].uw);
+    Ops<T>::sweep_axis(lv[q]->ny, S::ROWS, S::RING, grids[q].gy, grids[q].uh);
+    nz = std::max(nz, (lv[q]->nz + 1) / 2 * 2);
+    cells += (double)lv[q]->cells();
+  }
+  long best = -1;
+  int kchunk = nz;
+  for (int kc = nz; kc >= 2; kc -= 2) {
+    long nb = 0;
+    for (size_t q = 0; q < lv.size(); q++)
+      nb += (long)grids[q].gx * grids[q].gy * ((lv[q]->nz + kc - 1) / kc);
+    const long waves = (nb + cus - 1) / cus;
+    if (kc < nz && waves > 4 && waves > best) break;
+    const long cost = waves * ((kc + 2 * S::RING + S::NS) / S::NS);
+    if (best < 0 || cost <= best) {
+      best = cost;
+      kchunk = kc;
+    }
+  }
+  for (size_t q = 0; q < lv.size(); q++) {
+    grids[q].kchunk = kchunk;
+    grids[q].nch = (lv[q]->nz + kchunk - 1) / kchunk;
+  }
+  return cells / ((double)best * S::NS * cus * SW_COLS * S::ROWS);
+}
+
+// NIT iterations on level l of the given items in one launch of the sweep
+// kernel, swapping as above.  PRE: from x, from 0 or from x + P x_{l+1}.
+template <typename T, int NIT, int PRE>
+static void rec_sweep(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, const std::vector<int>& members, int l,
+                      T omega) {
+  using Sh = SweepShape<T, SW_WAVES, NIT, PRE>;
+  std::vector<const DevLevel<T>*> lv;
+  std::vector<SweepGrid> grids;
+  for (int i : members) lv.push_back(&H[i]->lv[l]);
+  sweep_grids<T, NIT, PRE>(lv, grids);
+  std::vector<SweepItem<T>> tab;
+  int nb = 0;
+  for (size_t q = 0; q < members.size(); q++) {
+    DevLevel<T>& d = H[members[q]]->lv[l];
+    SweepItem<T> e;
+    e.block0 = nb;
+    e.item = members[q];
+    e.A = Ops<T>::sweep_args(d, PRE == SW_PROLONG ? &H[members[q]]->lv[l + 1] : nullptr, omega);
+    e.A.G = grids[q];
+    nb += e.A.G.gx * e.A.G.gy * e.A.G.nch;
+    tab.push_back(e);
+    std::swap(d.x, d.x2);
+  }
+  const size_t off = S.put(tab);
+  const int n = (int)tab.size();
+  int* act = B->d_active;
+  const hipError_t rc = set_dynamic_lds((const void*)kb_sweep<T, NIT, PRE>, Sh::LDS * sizeof(T));
+  if (rc != hipSuccess) S.err = rc;
+  S.ops.push_back([=](hipStream_t st, const char* dev) {
+    hipLaunchKernelGGL((kb_sweep<T, NIT, PRE>), dim3((nb + 7) / 8 * 8), dim3(Sh::THREADS), Sh::LDS * sizeof(T), st,
+                       (const SweepItem<T>*)(dev + off), n, nb, act);
+  });
+}
+
+// the same by blocks of the levels in LDS
+template <typename T, typename Bl, int NIT, int PRE>
+static void rec_block(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, const std::vector<int>& members, int l,
+                      T omega) {
+  constexpr size_t lds = BlockShape<T, Bl, NIT, PRE>::LDS * sizeof(T);
+  std::vector<BlockItem<T>> tab;
+  int nb = 0;
+  for (int i : members) {
+    DevLevel<T>& d = H[i]->lv[l];
+    BlockItem<T> e;
+    e.block0 = nb;
+    e.item = i;
+    e.A = Ops<T>::template block_args<Bl>(d, PRE == SW_PROLONG ? &H[i]->lv[l + 1] : nullptr, omega);
+    nb += Ops<T>::template block_count<Bl>(d);
+    tab.push_back(e);
+    std::swap(d.x, d.x2);
+  }
+  const size_t off = S.put(tab);
+  const int n = (int)tab.size();
+  int* act = B->d_active;
+  const hipError_t rc = lds > 65536 ? set_dynamic_lds((const void*)kb_block<T, Bl, NIT, PRE>, lds) : hipSuccess;
+  if (rc != hipSuccess) S.err = rc;
+  S.ops.push_back([=](hipStream_t st, const char* dev) {
+    hipLaunchKernelGGL((kb_block<T, Bl, NIT, PRE>), dim3(nb), dim3(Bl::NT), lds, st,
+                       (const BlockItem<T>*)(dev + off), n, act);
+  });
+}
+
+// x_l += P x_{l+1}, for the given items
 template <typename T>
-static void rec_smooth(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, int l, int nu, T omega,
-                       bool zero_first) {
-  // tile shape per item: width 64 (FP64 always) or 128 (FP32), height 8, 16 or 32; unset, the
-  // single-grid solver's default for a level of this size
-  std::vector<int> g[2][3];
+static void rec_prolong(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, const std::vector<int>& members, int l) {
+  std::vector<ProlongItem<T>> tab;
+  int nb = 0;
+  for (int i : members) {
+    DevLevel<T>& f = H[i]->lv[l];
+    DevLevel<T>& c = H[i]->lv[l + 1];
+    ProlongItem<T> e;
+    e.block0 = nb;
+    e.item = i;
+    e.xf = f.x;
+    e.xc = c.x;
+    e.F = f.L();
+    e.C = c.L();
+    e.W = f.PW();
+    e.G = Ops<T>::prolong_grid(f, c);
+    nb += e.G.gx * e.G.gy * e.G.nch;
+    tab.push_back(e);
+  }
+  if (tab.empty()) return;
+  size_t off = S.put(tab);
+  int n = (int)tab.size();
+  int* act = B->d_active;
+  S.ops.push_back([=](hipStream_t st, const char* dev) {
+    hipLaunchKernelGGL((kb_prolong<T>), dim3(nb), dim3(MARCH_THREADS), 0, st, (const ProlongItem<T>*)(dev + off), n,
+                       act);
+  });
+}
+
+// How the iterations on level l of the items that have it (l < s) run: the
+// rules of the single-grid solver on the sum of the items' cells, which is
+// what fills the device.  Two at a time by the sweep kernel for items of
+// 100000 cells or more that have 4 M together (mixed batch of 18 items of
+// 32^3 to 192^3, 15 M cells: 5.9 ms without, 5.35 with those from 2 M cells
+// on, 4.85 from 800000, 4.5 from 100000; FP64 8.3, 8.2, 7.7 and 7.5 ms;
+// FP64, 16 items of 64^3: 3.37 ms without and 3.43 with); the others by blocks
+// up to the same sums as there (the 18 items, no sweeps: 6.2 ms in single
+// iterations, 5.9 with blocks on the coarser levels).  The rest one at a
+// time in the tiles set by the caller; unset, as the single-grid solver, but
+// for levels of 128 rows in FP32: 128 x 32 tiles leave the few blocks of the
+// items that take them alone on the device (two 128^3 items 41 us an
+// iteration; among the 64 x 8 blocks of the others they add 14).
+template <typename T>
+struct SmoothPlan {
+  std::vector<int> sweep, block, fused[2][3];   // fused: by tile width (64, 128) and height (8, 16, 32)
+  bool large = false;                           // block: BlockLarge
+  bool prolong_in_block = false;
+};
+
+template <typename T>
+static SmoothPlan<T> smooth_plan(pepsmg_batch* B, std::vector<Hier<T>*>& H, int l, int nu) {
+  SmoothPlan<T> P;
+  std::vector<int> rest;
+  std::vector<const DevLevel<T>*> lv;
+  long cells = 0;
   for (int i = 0; i < B->nitems; i++) {
     if (l >= B->items[i].s) continue;
+    const DevLevel<T>& d = H[i]->lv[l];
+    if (nu >= 2 && d.cells() >= 100000 && d.pxy * (long)sizeof(T) <= 0x7fffffffL) {
+      P.sweep.push_back(i);
+      lv.push_back(&d);
+      cells += d.cells();
+    } else {
+      rest.push_back(i);
+    }
+  }
+  if (!P.sweep.empty()) {
+    std::vector<SweepGrid> grids;
+    const double share = sweep_grids<T, 2, SW_X>(lv, grids);
+    if (cells < 4000000L || share < 0.15) {
+      rest.insert(rest.end(), P.sweep.begin(), P.sweep.end());
+      std::sort(rest.begin(), rest.end());
+      P.sweep.clear();
+    }
+  }
+  cells = 0;
+  for (int i : rest) cells += H[i]->lv[l].cells();
+  if (Ops<T>::blocks(cells)) {
+    P.block = rest;
+    P.large = Ops<T>::large_block(cells);
+    P.prolong_in_block = Ops<T>::prolong_in_block(cells);
+    return P;
+  }
+  for (int i : rest) {
     int tx = B->items[i].tile_x ? B->items[i].tile_x : B->opt.tile_x;
     int ty = B->items[i].tile_y ? B->items[i].tile_y : B->opt.tile_y;
-    if (!tx) tx = Ops<T>::default_tx(H[i]->lv[l]);
-    if (!ty) ty = Ops<T>::default_ty(H[i]->lv[l]);
-    int wx = (sizeof(T) == 4 && tx != 64) ? 1 : 0;
-    g[wx][ty == 32 ? 2 : ty == 16 ? 1 : 0].push_back(i);
+    const bool big = H[i]->lv[l].ny >= 256;
+    if (!tx) tx = big ? Ops<T>::FTX : 64;
+    if (!ty) ty = big ? 32 : 8;
+    P.fused[sizeof(T) == 4 && tx != 64][ty == 32 ? 2 : ty == 16 ? 1 : 0].push_back(i);
   }
-  for (int it = 0; it < nu; it++) {
-    bool z = zero_first && it == 0;
-    if (!g[0][0].empty()) rec_smooth_group<T, 64, 8>(B, S, H, g[0][0], l, z, omega);
-    if (!g[0][1].empty()) rec_smooth_group<T, 64, 16>(B, S, H, g[0][1], l, z, omega);
-    if (!g[0][2].empty()) rec_smooth_group<T, 64, 32>(B, S, H, g[0][2], l, z, omega);
+  return P;
+}
+
+// Record nu iterations on level l of every item that has it (per-level levels
+// only): from x, from x = 0 (zero) or from x + P x_{l+1} (prolong).
+template <typename T>
+static void rec_smooth(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, int l, int nu, T omega, bool zero,
+                       bool prolong) {
+  const SmoothPlan<T> P = smooth_plan<T>(B, H, l, nu);
+  // the launches that add the prolongation themselves
+  const bool ps = prolong && sizeof(T) == 4, pb = prolong && P.prolong_in_block;
+  if (prolong) {
+    std::vector<int> apart;
+    for (auto& w : P.fused)
+      for (auto& m : w) apart.insert(apart.end(), m.begin(), m.end());
+    if (!ps) apart.insert(apart.end(), P.sweep.begin(), P.sweep.end());
+    if (!pb) apart.insert(apart.end(), P.block.begin(), P.block.end());
+    rec_prolong<T>(B, S, H, apart, l);
+  }
+  auto fused = [&](const std::vector<int> (&g)[2][3], bool z) {
+    if (!g[0][0].empty()) rec_fused<T, 64, 8>(B, S, H, g[0][0], l, z, omega);
+    if (!g[0][1].empty()) rec_fused<T, 64, 16>(B, S, H, g[0][1], l, z, omega);
+    if (!g[0][2].empty()) rec_fused<T, 64, 32>(B, S, H, g[0][2], l, z, omega);
     if (sizeof(T) == 4) {
-      if (!g[1][0].empty()) rec_smooth_group<T, Ops<T>::FTX, 8>(B, S, H, g[1][0], l, z, omega);
-      if (!g[1][1].empty()) rec_smooth_group<T, Ops<T>::FTX, 16>(B, S, H, g[1][1], l, z, omega);
-      if (!g[1][2].empty()) rec_smooth_group<T, Ops<T>::FTX, 32>(B, S, H, g[1][2], l, z, omega);
+      if (!g[1][0].empty()) rec_fused<T, Ops<T>::FTX, 8>(B, S, H, g[1][0], l, z, omega);
+      if (!g[1][1].empty()) rec_fused<T, Ops<T>::FTX, 16>(B, S, H, g[1][1], l, z, omega);
+      if (!g[1][2].empty()) rec_fused<T, Ops<T>::FTX, 32>(B, S, H, g[1][2], l, z, omega);
     }
+  };
+  for (int it = 0; it < nu; it++) fused(P.fused, zero && it == 0);
+  if (!P.sweep.empty()) {
+    int it = 0;
+    for (; it + 2 <= nu; it += 2) {
+      if (it == 0 && zero) rec_sweep<T, 2, SW_ZERO>(B, S, H, P.sweep, l, omega);
+      else if (it == 0 && ps) {
+        if constexpr (sizeof(T) == 4) rec_sweep<T, 2, SW_PROLONG>(B, S, H, P.sweep, l, omega);
+      } else rec_sweep<T, 2, SW_X>(B, S, H, P.sweep, l, omega);
+    }
+    std::vector<int> g[2][3];
+    g[0][0] = P.sweep;
+    if (it < nu) fused(g, false);
+  }
+  if (!P.block.empty()) {
+    auto block = [&](auto Bc) {
+      using Bl = decltype(Bc);
+      for (int it = 0; it < nu; it += 2) {
+        const bool z = it == 0 && zero, p = it == 0 && pb;
+        if (nu - it >= 2) {
+          if (z) rec_block<T, Bl, 2, SW_ZERO>(B, S, H, P.block, l, omega);
+          else if (p) rec_block<T, Bl, 2, SW_PROLONG>(B, S, H, P.block, l, omega);
+          else rec_block<T, Bl, 2, SW_X>(B, S, H, P.block, l, omega);
+        } else {
+          if (z) rec_block<T, Bl, 1, SW_ZERO>(B, S, H, P.block, l, omega);
+          else if (p) rec_block<T, Bl, 1, SW_PROLONG>(B, S, H, P.block, l, omega);
+          else rec_block<T, Bl, 1, SW_X>(B, S, H, P.block, l, omega);
+        }
+      }
+    };
+    if (P.large) block(BlockLarge());
+    else block(BlockSmall());
   }
 }
 
@@ -391,37 +650,6 @@ static void rec_restrict(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, in
   });
 }
 
-// x_l += P x_{l+1}, for items with l < s
-template <typename T>
-static void rec_prolong(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, int l) {
-  std::vector<ProlongItem<T>> tab;
-  int nb = 0;
-  for (int i = 0; i < B->nitems; i++) {
-    if (l >= B->items[i].s) continue;
-    DevLevel<T>& f = H[i]->lv[l];
-    DevLevel<T>& c = H[i]->lv[l + 1];
-    ProlongItem<T> e;
-    e.block0 = nb;
-    e.item = i;
-    e.xf = f.x;
-    e.xc = c.x;
-    e.F = f.L();
-    e.C = c.L();
-    e.W = f.PW();
-    e.G = Ops<T>::prolong_grid(f, c);
-    nb += e.G.gx * e.G.gy * e.G.nch;
-    tab.push_back(e);
-  }
-  if (tab.empty()) return;
-  size_t off = S.put(tab);
-  int n = (int)tab.size();
-  int* act = B->d_active;
-  S.ops.push_back([=](hipStream_t st, const char* dev) {
-    hipLaunchKernelGGL((kb_prolong<T>), dim3(nb), dim3(MARCH_THREADS), 0, st, (const ProlongItem<T>*)(dev + off), n,
-                       act);
-  });
-}
-
 template <typename T>
 static void rec_coarse(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, int nu, int nu_post, T omega,
                        double tol) {
@@ -448,13 +676,12 @@ static void rec_vcycle(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, int 
   int D = 0;
   for (auto& it : B->items) D = std::max(D, it.s);
   for (int l = 0; l < D; l++) {
-    rec_smooth<T>(B, S, H, l, nu, omega, l > 0 || fine_zero);
+    rec_smooth<T>(B, S, H, l, nu, omega, l > 0 || fine_zero, false);
     rec_restrict<T>(B, S, H, l);
   }
   rec_coarse<T>(B, S, H, nu, nu_post, omega, tol);
   for (int l = D - 1; l >= 0; l--) {
-    rec_prolong<T>(B, S, H, l);
-    rec_smooth<T>(B, S, H, l, nu_post, omega, false);
+    rec_smooth<T>(B, S, H, l, nu_post, omega, false, true);
   }
 }
 
@@ -712,6 +939,8 @@ static int batch_build(pepsmg_batch* B, int nu, double tol, double omega) {
     rec_resid<0>(B, S, false);
     rec_check(B, S, tol, maxsteps, 0);
   }
+  HIP_TRY(B->sched[0].err);
+  HIP_TRY(B->sched[1].err);
   // the recorders swapped pointers as the launches will; FP64 cycles swap an
   // even number of times, the mixed pair of steps too
   size_t total = 0;

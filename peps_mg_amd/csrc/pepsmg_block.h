@@ -56,8 +56,9 @@ struct BlockShape {
   static constexpr int LDS = 2 * NPAIR + NW + (PRE == SW_PROLONG ? NW + NC : 0);   // elements
 };
 
+// tile `bid` of the level
 template <typename T, typename B, int NIT, int PRE, bool NORM>
-__global__ void __launch_bounds__(B::NT) k_block(BlockArgs<T> A) {
+__device__ __forceinline__ void block_tile(const BlockArgs<T>& A, int bid) {
   using S = BlockShape<T, B, NIT, PRE>;
   using V2 = typename SwPair<T>::type;
   constexpr bool F64 = sizeof(T) == 8;
@@ -72,7 +73,7 @@ __global__ void __launch_bounds__(B::NT) k_block(BlockArgs<T> A) {
 
   const Lvl<T>& L = A.L;
   const int t = threadIdx.x;
-  const int bx = blockIdx.x % A.gx, byz = blockIdx.x / A.gx;
+  const int bx = bid % A.gx, byz = bid / A.gx;
   const int i0 = 1 + bx * B::BX - H, j0 = 1 + (byz % A.gy) * B::BY - H, k0 = 1 + (byz / A.gy) * B::BZ - H;   // i0 odd
 
   // ---- all loads ----
@@ -218,7 +219,7 @@ __global__ void __launch_bounds__(B::NT) k_block(BlockArgs<T> A) {
     }
     __shared__ double sh[NT / 64];
     const double s = block_sum(acc, sh);             // (its barriers also close the reads of x_in)
-    if (t == 0) A.partial[blockIdx.x] = s;
+    if (t == 0) A.partial[bid] = s;
   }
 #pragma unroll
   for (int s = 1; s <= 2 * NIT; s++) {
@@ -255,6 +256,11 @@ __global__ void __launch_bounds__(B::NT) k_block(BlockArgs<T> A) {
       else u[0] = o.x;
     }
   }
+}
+
+template <typename T, typename B, int NIT, int PRE, bool NORM>
+__global__ void __launch_bounds__(B::NT) k_block(BlockArgs<T> A) {
+  block_tile<T, B, NIT, PRE, NORM>(A, blockIdx.x);
 }
 
 }  // namespace pepsmg

@@ -348,12 +348,9 @@ struct Ops {
     return share >= 0.15;
   }
 
-  // NIT red/black iterations on level d in one pass, x -> x2, then swap.
-  // PRE: from x, from 0, or from x + P x_c (c the next coarser level, every
-  // axis halving).  to_caller (FP64): the caller's solution also receives x.
-  template <int NIT, int PRE>
-  void sweep(DevLevel<T>& d, const DevLevel<T>* c, T omega, bool to_caller = false) {
-    using S = SweepShape<T, SW_WAVES, NIT, PRE>;
+  // arguments of a k_sweep launch (x -> x2) but for its grid; c: the coarser
+  // level of SW_PROLONG, or null
+  static SweepArgs<T> sweep_args(const DevLevel<T>& d, const DevLevel<T>* c, T omega) {
     SweepArgs<T> A;
     std::memset(&A, 0, sizeof A);
     A.xo = d.x2;
@@ -365,11 +362,21 @@ struct Ops {
     A.zhi = d.zhi;
     A.c5u = d.c5u;
     A.c6u = d.c6u;
-    if (PRE == SW_PROLONG) {
+    if (c) {
       A.xc = c->x;
       A.C = c->L();
       A.W = d.PW();
     }
+    return A;
+  }
+
+  // NIT red/black iterations on level d in one pass, x -> x2, then swap.
+  // PRE: from x, from 0, or from x + P x_c (c the next coarser level, every
+  // axis halving).  to_caller (FP64): the caller's solution also receives x.
+  template <int NIT, int PRE>
+  void sweep(DevLevel<T>& d, const DevLevel<T>* c, T omega, bool to_caller = false) {
+    using S = SweepShape<T, SW_WAVES, NIT, PRE>;
+    SweepArgs<T> A = sweep_args(d, c, omega);
     if (to_caller) {
       A.ext = caller_sol;
       A.U = caller_lvl;
@@ -392,11 +399,41 @@ struct Ops {
   // blocks on its 128^3 level, 128^3 takes 2.99 against 2.81); mixed 32^3 0.59
   // against 0.70 ms, 64^3 0.80 against 0.99, 96^3 1.05 against 1.31, 128^3
   // 1.47 against 1.54.
-  static bool blocks(const DevLevel<T>& d) { return d.cells() <= (sizeof(T) == 8 ? 1200000L : 3000000L); }
+  static bool blocks(long cells) { return cells <= (sizeof(T) == 8 ? 1200000L : 3000000L); }
+  static bool blocks(const DevLevel<T>& d) { return blocks(d.cells()); }
   // 32 x 8 x 8 blocks of 1024 threads from 150000 cells on: less ring per cell
   // (96^3 FP64 2.14 against 2.38 ms); below, 16 x 8 x 4 keeps more CUs busy
   // (64^3 FP64 1.56 against 1.69 ms when its fine level, too, takes them)
-  static bool large_block(const DevLevel<T>& d) { return d.cells() > (sizeof(T) == 8 ? 300000L : 150000L); }
+  static bool large_block(long cells) { return cells > (sizeof(T) == 8 ? 300000L : 150000L); }
+  // The prolongation in the launch works on the whole ring: it pays up to
+  // 200000 cells (96^3 FP64 2.11 ms with it on the fine level, 2.00 without;
+  // mixed 128^3 1.45 and 1.36).
+  static bool prolong_in_block(long cells) { return cells <= 200000L; }
+
+  // arguments of a k_block launch (x -> x2) with blocks B, and their number;
+  // c as for sweep_args
+  template <typename B>
+  static BlockArgs<T> block_args(const DevLevel<T>& d, const DevLevel<T>* c, T omega) {
+    BlockArgs<T> A;
+    std::memset(&A, 0, sizeof A);
+    A.xo = d.x2;
+    A.xi = d.x;
+    A.b = d.b;
+    A.L = d.L();
+    A.omega = omega;
+    if (c) {
+      A.xc = c->x;
+      A.C = c->L();
+      A.W = d.PW();
+    }
+    A.gx = (d.nx + B::BX - 1) / B::BX;
+    A.gy = (d.ny + B::BY - 1) / B::BY;
+    return A;
+  }
+  template <typename B>
+  static int block_count(const DevLevel<T>& d) {
+    return (d.nx + B::BX - 1) / B::BX * ((d.ny + B::BY - 1) / B::BY) * ((d.nz + B::BZ - 1) / B::BZ);
+  }
 
   // NIT iterations on level d by blocks, x -> x2, then swap (PRE, c,
   // to_caller as for sweep).  NORM (FP64, from x): the blocks' partial sums of
@@ -404,26 +441,14 @@ struct Ops {
   template <typename B, int NIT, int PRE, bool NORM = false>
   int block_launch(DevLevel<T>& d, const DevLevel<T>* c, T omega, bool to_caller, double* partial, T* out) {
     using S = BlockShape<T, B, NIT, PRE>;
-    BlockArgs<T> A;
-    std::memset(&A, 0, sizeof A);
-    A.xo = out ? out : d.x2;
-    A.xi = d.x;
-    A.b = d.b;
-    A.L = d.L();
-    A.omega = omega;
-    if (PRE == SW_PROLONG) {
-      A.xc = c->x;
-      A.C = c->L();
-      A.W = d.PW();
-    }
+    BlockArgs<T> A = block_args<B>(d, c, omega);
+    if (out) A.xo = out;
     if (to_caller) {
       A.ext = caller_sol;
       A.U = caller_lvl;
     }
     A.partial = partial;
-    A.gx = (d.nx + B::BX - 1) / B::BX;
-    A.gy = (d.ny + B::BY - 1) / B::BY;
-    const int nb = A.gx * A.gy * ((d.nz + B::BZ - 1) / B::BZ);
+    const int nb = block_count<B>(d);
     bool timed;
     timer_begin(d, 0, timed);
     if (S::LDS * sizeof(T) > 65536) set_dynamic_lds((const void*)k_block<T, B, NIT, PRE, NORM>, S::LDS * sizeof(T));
@@ -436,7 +461,7 @@ struct Ops {
   template <int NIT, int PRE, bool NORM = false>
   int block(DevLevel<T>& d, const DevLevel<T>* c, T omega, bool to_caller = false, double* partial = nullptr,
             T* out = nullptr) {
-    return large_block(d) ? block_launch<BlockLarge, NIT, PRE, NORM>(d, c, omega, to_caller, partial, out)
+    return large_block(d.cells()) ? block_launch<BlockLarge, NIT, PRE, NORM>(d, c, omega, to_caller, partial, out)
                           : block_launch<BlockSmall, NIT, PRE, NORM>(d, c, omega, to_caller, partial, out);
   }
 
@@ -444,10 +469,7 @@ struct Ops {
   void iterate_blocks(DevLevel<T>& d, T omega, int nu, bool zero_start, DevLevel<T>* c, int last_mode) {
     int it = 0;
     auto last = [&](int n) { return it + n == nu && last_mode == 4; };
-    // the prolongation in the launch works on the whole ring: it pays up to
-    // 200000 cells (96^3 FP64 2.11 ms with it on the fine level, 2.00 without;
-    // mixed 128^3 1.45 and 1.36)
-    if (c && !(d.ps[0] == 2 && d.ps[1] == 2 && d.ps[2] == 2 && d.cells() <= 200000)) {
+    if (c && !(d.ps[0] == 2 && d.ps[1] == 2 && d.ps[2] == 2 && prolong_in_block(d.cells()))) {
       prolong_add(d, *c, d.x);
       c = nullptr;
     }

@@ -128,8 +128,15 @@ struct SweepShape {
   static constexpr int LDS = 2 * RING * EDGE + (NBR + NBB) * R * THREADS;   // elements
 };
 
+// Block number of the level, or of all levels of a launch, that blockIdx
+// stands for: contiguous eighths of the tiles (x fastest, then y, then
+// chunks) per XCD, so that neighbouring tiles re-read each other's rings from
+// the XCD's L2.  The grid is rounded up to a multiple of 8.
+__device__ __forceinline__ int sweep_block() { return (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3); }
+
+// block `lin` of the level
 template <typename T, int W, int NIT, int PRE>
-__global__ void __launch_bounds__(64 * W) k_sweep(SweepArgs<T> A) {
+__device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
   using S = SweepShape<T, W, NIT, PRE>;
   using V2 = typename SwPair<T>::type;
   constexpr bool F64 = sizeof(T) == 8;
@@ -143,11 +150,7 @@ __global__ void __launch_bounds__(64 * W) k_sweep(SweepArgs<T> A) {
 
   const Lvl<T>& L = A.L;
   const SweepGrid& G = A.G;
-  // contiguous eighths of the tiles (x fastest, then y, then chunks) per XCD:
-  // neighbouring tiles re-read each other's rings from the XCD's L2
-  const int ntile = G.gx * G.gy, nb = ntile * G.nch;
-  const int lin = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  if (lin >= nb) return;                             // the grid is rounded up to a multiple of 8
+  const int ntile = G.gx * G.gy;
   const int bz = lin / ntile, tile = lin - bz * ntile;
   const int ty = tile / G.gx, tx = tile - ty * G.gx;
   const int us = 1 + tx * G.uw, ue = min(us + G.uw - 1, L.nx);   // columns / rows stored
@@ -538,6 +541,12 @@ __global__ void __launch_bounds__(64 * W) k_sweep(SweepArgs<T> A) {
     }
     m += NS;
   }
+}
+
+template <typename T, int W, int NIT, int PRE>
+__global__ void __launch_bounds__(64 * W) k_sweep(SweepArgs<T> A) {
+  const int lin = sweep_block();
+  if (lin < A.G.gx * A.G.gy * A.G.nch) sweep_tile<T, W, NIT, PRE>(A, lin);
 }
 
 }  // namespace pepsmg
