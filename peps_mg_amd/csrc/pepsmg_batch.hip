@@ -509,7 +509,7 @@ static void rec_prolong(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, con
 template <typename T>
 struct SmoothPlan {
   std::vector<int> sweep, block, fused[2][3];   // fused: by tile width (64, 128) and height (8, 16, 32)
-  bool large = false;                           // block: BlockLarge
+  int shape = 0;                                // block: BlockSmall, BlockLarge (1), BlockTall (2)
   bool prolong_in_block = false;
 };
 
@@ -543,8 +543,8 @@ static SmoothPlan<T> smooth_plan(pepsmg_batch* B, std::vector<Hier<T>*>& H, int 
   for (int i : rest) cells += H[i]->lv[l].cells();
   if (Ops<T>::blocks(cells)) {
     P.block = rest;
-    P.large = Ops<T>::large_block(cells);
     P.prolong_in_block = Ops<T>::prolong_in_block(cells);
+    P.shape = Ops<T>::tall_block(cells) ? 2 : Ops<T>::large_block(cells) ? 1 : 0;
     return P;
   }
   for (int i : rest) {
@@ -613,8 +613,9 @@ static void rec_smooth(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, int 
         }
       }
     };
-    if (P.large) block(BlockLarge());
-    else block(BlockSmall());
+    if (P.shape == 0) block(BlockSmall());
+    else if (P.shape == 1) block(BlockLarge());
+    else if constexpr (sizeof(T) == 4) block(BlockTall());
   }
 }
 

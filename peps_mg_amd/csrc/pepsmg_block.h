@@ -43,6 +43,10 @@ struct BlockTile {
 };
 using BlockSmall = BlockTile<16, 8, 4, 512>;
 using BlockLarge = BlockTile<32, 8, 8, 1024>;
+// (Its 8 pairs a thread take 127 registers.  One word of state per pair instead
+// of four brings BlockLarge to 64, for two blocks on a CU, but unpacking costs
+// what that gains: the half-sweeps are short of instruction slots.)
+using BlockTall = BlockTile<32, 16, 8, 1024>;
 
 template <typename T, typename B, int NIT, int PRE>
 struct BlockShape {

@@ -405,6 +405,13 @@ struct Ops {
   // (96^3 FP64 2.14 against 2.38 ms); below, 16 x 8 x 4 keeps more CUs busy
   // (64^3 FP64 1.56 against 1.69 ms when its fine level, too, takes them)
   static bool large_block(long cells) { return cells > (sizeof(T) == 8 ? 300000L : 150000L); }
+  // FP32 from 400000 cells on: 32 x 16 x 8, where a cell's share of the ring
+  // shrinks further (mixed 80^3 0.972 against 0.945 ms, 96^3 1.020 against
+  // 0.977, 128^3 1.39 against 1.32, 256^3, on its 128^3 level, 3.12 against
+  // 3.03; also on 64^3 levels 128^3 takes 1.37).  64 x 8 x 8 and 32 x 16 x 16
+  // are slower (128^3 1.31 and 1.53 when this one took 1.29), and in FP64 no
+  // other shape gains.
+  static bool tall_block(long cells) { return sizeof(T) == 4 && cells > 400000L; }
   // The prolongation in the launch works on the whole ring: it pays up to
   // 200000 cells (96^3 FP64 2.11 ms with it on the fine level, 2.00 without;
   // mixed 128^3 1.45 and 1.36).
@@ -461,6 +468,8 @@ struct Ops {
   template <int NIT, int PRE, bool NORM = false>
   int block(DevLevel<T>& d, const DevLevel<T>* c, T omega, bool to_caller = false, double* partial = nullptr,
             T* out = nullptr) {
+    if constexpr (sizeof(T) == 4 && PRE != SW_PROLONG && !NORM)
+      if (tall_block(d.cells())) return block_launch<BlockTall, NIT, PRE, NORM>(d, c, omega, to_caller, partial, out);
     return large_block(d.cells()) ? block_launch<BlockLarge, NIT, PRE, NORM>(d, c, omega, to_caller, partial, out)
                           : block_launch<BlockSmall, NIT, PRE, NORM>(d, c, omega, to_caller, partial, out);
   }

@@ -59,3 +59,17 @@ def test_vcycle_bitwise(dims, nlevel, nu):
     assert np.max(np.abs(res.history - hist)) <= 1e-12
     assert np.array_equal(d_x.cpu().numpy(), xo)
     mg.destroy()
+
+
+@pytest.mark.parametrize("dims", [(96, 80, 56), (97, 81, 57), (95, 79, 63)])
+@pytest.mark.parametrize("omega,nu", [(1.0, 1), (1.6, 2), (1.0, 5)])
+def test_fp32_tall_tiles(dims, omega, nu):
+    """FP32 levels of 32 x 16 x 8 tiles, within the bound above."""
+    g = O.Grid(*dims, a=tuple(1.03 if d % 2 == 0 else 1.0 for d in dims))   # (odd axes cannot be stretched)
+    A = g.matrix()
+    x = O.uniform_field(*dims, 24).astype(np.float32).astype(np.float64)
+    b = O.uniform_field(*dims, 25).astype(np.float32).astype(np.float64)
+    xo = x.copy()
+    rbgs_iterator_fp32(x, b, sdm_from(g), nu, omega)
+    O.rbgs_iterator(xo, A, b, nu, omega)
+    assert np.abs(x - xo).max() <= 1e-6 * (1 + nu) * np.abs(xo).max()
