@@ -233,12 +233,17 @@ __host__ __device__ inline int pc_stage_elems(int nx, int ny, int nz, bool trans
 
 // copies level G's arrays (and transfer weights when R, P are given) to s.
 // Every load of a thread is issued before its first LDS store (clamped
-// indices, no branch next to a load), so staging costs one load latency.
+// indices, no branch next to a load), so staging costs one load latency;
+// threads from `first` on begin, and first moves to the next wave behind
+// them, so that the levels' latencies overlap (a 16^3 level and three below
+// it, with b: 5.7 us one level after the other).
 template <typename T>
-__device__ void pc_stage(T* s, const Lvl<T>& G, const RestrictW<T>* R, const ProlongW<T>* P) {
+__device__ void pc_stage(T* s, const Lvl<T>& G, const RestrictW<T>* R, const ProlongW<T>* P, int& first) {
   const int ex = G.nx + 2, ey = G.ny + 2, ez = G.nz + 2;
   const int em = max(ex, max(ey, ez));
-  for (int c = threadIdx.x; c < em; c += blockDim.x) {
+  const int t = ((int)threadIdx.x - first) & (PC_THREADS - 1);
+  first = (first + em + 63) & ~63 & (PC_THREADS - 1);
+  for (int c = t; c < em; c += PC_THREADS) {
     const int cx = min(c, ex - 1), cy = min(c, ey - 1), cz = min(c, ez - 1);
     T v[15];
     v[0] = G.cwx[cx];
@@ -756,9 +761,63 @@ __device__ void pc_restrict(TC* bc, T* r, const T* x, const T* b, const Lvl<T>& 
   __syncthreads();
 }
 
-// x_f += P x_c (prolong_at's weights, terms and order) on a compact level
+// x_f += P x_c (prolong_at's weights, terms and order) on a compact level that
+// halves every axis, by pairs of fine cells (i odd, i + 1) with one parent:
+// they share the rows' indices and weights and the parent's
+// values.  What a cell costs is instructions (onto 16^3, cell by cell, 8.4 us
+// of a 54 us FP64 kernel; by pairs 49 in all, FP32 36 and 29 us, staging
+// included).
+template <typename T>
+__device__ void pc_prolong_pairs(T* xf, const T* xc, const Lvl<T>& F, const Lvl<T>& C, const ProlongW<T>& W) {
+  const int hx = C.nx, np = hx * F.ny * F.nz;
+  const unsigned long long mh = pc_magic(hx), my = pc_magic(F.ny);
+  for (int p = threadIdx.x; p < np; p += blockDim.x) {
+    const int row = pc_div(p, mh), kk = pc_div(row, my);
+    const int ci = p - row * hx, j = row - kk * F.ny + 1, k = kk + 1, i = 2 * ci + 1;   // ci from 0
+    const bool jo = j & 1, ko = k & 1;
+    const T sy = jo ? W.py_[j] : W.ny_[j], ny = jo ? W.py_[j + 1] : W.ny_[j - 1];
+    const T sz = ko ? W.pz_[k] : W.nz_[k], nz = ko ? W.pz_[k + 1] : W.nz_[k - 1];
+    const int cj = (j - 1) >> 1, ck = (k - 1) >> 1, nj = jo ? cj - 1 : cj + 1, nk = ko ? ck - 1 : ck + 1;   // from 0
+    const bool vy = nj >= 0 && nj < C.ny, vz = nk >= 0 && nk < C.nz;
+    const bool vw = ci > 0, ve = ci + 1 < hx;
+    const int ow = vw ? -1 : 0, oe = ve ? 1 : 0;
+    const T* a = xc + ci + hx * (cj + C.ny * ck);
+    const T* rows[4] = {a, a + (vy ? hx * (nj - cj) : 0), a + (vz ? hx * C.ny * (nk - ck) : 0),
+                        a + (vy && vz ? hx * (nj - cj + C.ny * (nk - ck)) : 0)};
+    const bool in[4] = {true, vy, vz, vy && vz};
+    T w[4], m[4], e[4];                              // west of the parent's column, in it, east of it
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      w[r] = rows[r][ow];
+      m[r] = rows[r][0];
+      e[r] = rows[r][oe];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      w[r] = in[r] && vw ? w[r] : T(0);
+      m[r] = in[r] ? m[r] : T(0);
+      e[r] = in[r] && ve ? e[r] : T(0);
+    }
+    T* x = xf + 2 * p;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const T sx = c ? W.nx_[i + 1] : W.px_[i], nx = c ? W.nx_[i] : W.px_[i + 1];
+      const T* o = c ? e : w;
+      const T num = sx * sy * sz * m[0] + nx * sy * sz * o[0] + sx * ny * sz * m[1] + sx * sy * nz * m[2] +
+                    nx * ny * sz * o[1] + nx * sy * nz * o[2] + sx * ny * nz * m[3] + nx * ny * nz * o[3];
+      x[c] = x[c] + num / ((sx + nx) * (sy + ny) * (sz + nz));
+    }
+  }
+  __syncthreads();
+}
+
+// x_f += P x_c on any compact level
 template <typename T>
 __device__ void pc_prolong_add(T* xf, const T* xc, const Lvl<T>& F, const Lvl<T>& Cc, const ProlongW<T>& W) {
+  if (W.sx == 2 && W.sy == 2 && W.sz == 2 && F.nx == 2 * Cc.nx && F.ny == 2 * Cc.ny && F.nz == 2 * Cc.nz) {
+    pc_prolong_pairs(xf, xc, F, Cc, W);
+    return;
+  }
   const int n = F.nx * F.ny * F.nz;
   const unsigned long long mx = pc_magic(F.nx), my = pc_magic(F.ny);
   auto V = [&](int a, int bb, int cc) -> T {
@@ -801,24 +860,29 @@ __device__ __forceinline__ void coarse_vcycle_block(const PCArgs<T>& A) {
   __shared__ double seq[64];
   const int top = A.nlev - 1;                     // index of the coarsest level
   // coefficients and transfer weights into LDS, b_s from global
-  for (int q = 0; q < top; q++) pc_stage(sm + A.coff[q], A.lv[q], &A.rw[q], &A.pw[q]);
-  pc_stage(smd + A.ccoff, A.lc, (const RestrictW<double>*)nullptr, (const ProlongW<double>*)nullptr);
   {
-    // four loads in flight per thread (clamped cells) before the LDS stores
     const Lvl<T>& L = A.lv[0];
     const int n = L.nx * L.ny * L.nz;
-    const int bd = blockDim.x;
-    for (int c0 = threadIdx.x; c0 < n; c0 += 4 * bd) {
-      T v[4];
+    const unsigned long long mx = pc_magic(L.nx), my = pc_magic(L.ny);
+    // four loads in flight per thread (clamped cells) before the LDS stores
+    T v[4];
+    auto load = [&](int c0) {
 #pragma unroll
       for (int u = 0; u < 4; u++) {
-        const int c = min(c0 + u * bd, n - 1);
-        const int i = c % L.nx + 1, j = (c / L.nx) % L.ny + 1, k = c / (L.nx * L.ny) + 1;
-        v[u] = A.gbs[lidx(A.gl, i, j, k)];
+        const int c = min(c0 + u * PC_THREADS, n - 1);
+        const int row = pc_div(c, mx), kk = pc_div(row, my);
+        v[u] = A.gbs[lidx(A.gl, c - row * L.nx + 1, row - kk * L.ny + 1, kk + 1)];
       }
+    };
+    load(threadIdx.x);
+    int first = 0;
+    for (int q = 0; q < top; q++) pc_stage(sm + A.coff[q], A.lv[q], &A.rw[q], &A.pw[q], first);
+    pc_stage(smd + A.ccoff, A.lc, (const RestrictW<double>*)nullptr, (const ProlongW<double>*)nullptr, first);
+    for (int c0 = threadIdx.x; c0 < n; c0 += 4 * PC_THREADS) {
+      if (c0 >= 4 * PC_THREADS) load(c0);
 #pragma unroll
       for (int u = 0; u < 4; u++) {
-        const int c = c0 + u * bd;
+        const int c = c0 + u * PC_THREADS;
         if (c < n) {
           if (top == 0) smd[A.bcoff + c] = (double)v[u];
           else sm[A.boff[0] + c] = v[u];
