@@ -664,7 +664,7 @@ struct PCPair {
       c2[h] = L.cex[is];
       c0[h] = diag(c1[h], c2[h], c3, c4, c5, c6);
       rc[h] = T(1) / c0[h];
-      bv[h] = bs[q[h]];
+      bv[h] = bs ? bs[q[h]] : T(0);
       if constexpr (sizeof(T) == 8) kept = kept && kd_divisor(c0[h]);
     }
   }

@@ -137,12 +137,127 @@ k_cg_p(T* __restrict__ p, const T* __restrict__ r, const double* __restrict__ sc
   });
 }
 
+// All nu CG iterations on a level of up to PC_PAIRS PC_THREADS pairs (i odd,
+// i + 1) by one workgroup: x and r in registers, the direction p in LDS, the
+// scalars formed by every thread from the waves' sums.  Bound: latency.  The
+// separate kernels take 8 and 4 us an iteration on levels of 16^3 and 8^3,
+// whose cells a few blocks cover; here an iteration is two barriers for its
+// sums and one for p.  Values are those of the separate kernels but for the
+// order of the sums.
+template <typename T>
+__global__ void __launch_bounds__(PC_THREADS)
+k_cg_small(T* __restrict__ x, const T* __restrict__ b, Lvl<T> L, int nu, int zero_x) {
+  __shared__ T ps[2 * PC_PAIRS * PC_THREADS + 2];   // the level's cells and the two zeros beside them
+  __shared__ double part[2][PC_THREADS / 64];
+  const int hx = (L.nx + 1) / 2, np = hx * L.ny * L.nz, nc = L.nx * L.ny * L.nz;
+  const unsigned long long mh = pc_magic(hx), my = pc_magic(L.ny);
+  PCPair<T> P[PC_PAIRS];
+  long g[PC_PAIRS];                                  // the pair's first cell in x and b
+  T xv[PC_PAIRS][2], rv[PC_PAIRS][2], pv[PC_PAIRS][2], av[PC_PAIRS][2];   // cells in PCPair's order
+  if (threadIdx.x < 2) ps[nc + threadIdx.x] = T(0);
+#pragma unroll
+  for (int u = 0; u < PC_PAIRS; u++) {
+    const int p = threadIdx.x + u * PC_THREADS, pp = p < np ? p : 0;
+    const int row = pc_div(pp, mh), kk = pc_div(row, my);
+    g[u] = lidx(L, 1 + 2 * (pp - row * hx), row - kk * L.ny + 1, kk + 1);
+    P[u].load(L, (const T*)nullptr, p, mh, my);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const bool in = P[u].in[h];
+      const long q = g[u] + (in ? P[u].o[h] : 0);
+      P[u].bv[h] = b[q];
+      xv[u][h] = in && !zero_x ? x[q] : T(0);
+      if (in) ps[P[u].q[h]] = xv[u][h];
+    }
+  }
+  __syncthreads();
+  // (A p)(cell h of pair u) from ps
+  auto apply = [&](int u, int h) -> T {
+    const PCPair<T>& c = P[u];
+    const int o = c.o[h];
+    return c.c0[h] * ps[c.q[h]] + c.c1[h] * ps[c.w[h]] + c.c2[h] * ps[c.e[h]] + c.c3 * ps[c.s + o] +
+           c.c4 * ps[c.n + o] + c.c5 * ps[c.b + o] + c.c6 * ps[c.t + o];
+  };
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  auto sum = [&](double v, int slot) {               // over the block, on every thread
+    v = pc_wave_sum(v);
+    if (lane == 0) part[slot][wave] = v;
+    __syncthreads();
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < PC_THREADS / 64; w++) t += part[slot][w];
+    return t;
+  };
+  // r = b - A x, p = r, (r, r)  (:196-204)
+  double acc = 0.0;
+#pragma unroll
+  for (int u = 0; u < PC_PAIRS; u++) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      rv[u][h] = P[u].in[h] ? P[u].bv[h] - (zero_x ? T(0) : apply(u, h)) : T(0);
+      pv[u][h] = rv[u][h];
+      acc += (double)rv[u][h] * (double)rv[u][h];
+    }
+  }
+  double rr = sum(acc, 0);                           // (its barrier also closes the reads of x)
+  for (int it = 0; it < nu; it++) {
+#pragma unroll
+    for (int u = 0; u < PC_PAIRS; u++) {
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        if (P[u].in[h]) ps[P[u].q[h]] = pv[u][h];
+    }
+    __syncthreads();
+    acc = 0.0;
+#pragma unroll
+    for (int u = 0; u < PC_PAIRS; u++) {
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        av[u][h] = P[u].in[h] ? apply(u, h) : T(0);
+        acc += (double)av[u][h] * (double)pv[u][h];
+      }
+    }
+    const T alpha = (T)(rr / sum(acc, 1));           // :206-209
+    acc = 0.0;
+#pragma unroll
+    for (int u = 0; u < PC_PAIRS; u++) {
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        if (!P[u].in[h]) continue;
+        xv[u][h] = xv[u][h] + alpha * pv[u][h];      // :210-216
+        rv[u][h] = rv[u][h] - alpha * av[u][h];
+        acc += (double)rv[u][h] * (double)rv[u][h];
+      }
+    }
+    if (it + 1 == nu) break;
+    const double rn = sum(acc, 0);                   // :221
+    const T beta = (T)(rn / rr);
+    rr = rn;
+#pragma unroll
+    for (int u = 0; u < PC_PAIRS; u++) {
+#pragma unroll
+      for (int h = 0; h < 2; h++) pv[u][h] = rv[u][h] + beta * pv[u][h];   // :223-229
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < PC_PAIRS; u++) {
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+      if (P[u].in[h]) x[g[u] + P[u].o[h]] = xv[u][h];
+  }
+}
+
 // p2: a second direction buffer (with the march kernels the direction
 // update of iteration it-1 is folded into iteration it's A p launch, which
 // writes the new direction there; p and p2 then trade places)
 template <typename T>
 static void cg_iterate(Ops<T>& op, DevLevel<T>& d, T* x, const T* b, T* r, T* p, T* p2, T* ap, int nu, bool zero_x,
                        double* partial, double* sc) {
+  // levels that one workgroup holds (a 128^3 CG(4) solve 6.58 against 5.45 ms)
+  if (nu > 0 && (long)((d.nx + 1) / 2) * d.ny * d.nz <= PC_PAIRS * PC_THREADS) {
+    hipLaunchKernelGGL((k_cg_small<T>), dim3(1), dim3(PC_THREADS), 0, op.s, x, b, d.L(), nu, zero_x ? 1 : 0);
+    return;
+  }
   const long nrow = (long)d.ny * d.nz;
   const int eb = (int)std::max(1L, std::min<long>((nrow + CG_WAVES - 1) / CG_WAVES, RED_BLOCKS));
   const dim3 eblk(64 * CG_WAVES);
