@@ -62,6 +62,12 @@ struct Ops {
     return cache[key] = per * cus;
   }
 
+  // nxy tiles split into chunks of at least 4 planes fill the device's
+  // resident blocks exactly
+  static bool one_wave(const DevLevel<T>& d, long nxy, int resident_blocks) {
+    return resident_blocks > 0 && resident_blocks % nxy == 0 && d.nz / (resident_blocks / nxy) >= 4;
+  }
+
   // Block decomposition of the fused smoother: TX x TY tiles marching
   // through z-chunks (even, so every chunk starts on an odd plane).  When
   // the tiles divide the resident block count, one chunk count fills the
@@ -81,7 +87,7 @@ struct Ops {
     G.gy = (d.ny + TY - 1) / TY;
     long nxy = (long)G.gx * G.gy;
     long nch;
-    if (resident_blocks > 0 && resident_blocks % nxy == 0 && d.nz / (resident_blocks / nxy) >= 4) {
+    if (one_wave(d, nxy, resident_blocks)) {
       nch = resident_blocks / nxy;
     } else {
       const int min_planes = batched ? 4 : 2, long_from = batched ? 96 : 192;
@@ -196,17 +202,24 @@ struct Ops {
   // tile sizes in use: width 64 cells in FP64 and 128 in FP32 (the same
   // bytes per row) unless set
   int tile_x = 0;
-  // Unless set, the tile follows the level: on levels of 256 rows or more
-  // 64 x 32 (FP64) and 128 x 32 (FP32), below 64 x 8, whose smaller blocks
-  // keep more CUs busy (FP32 solves: 256^3 4.6 against 5.2 ms, 128^3 2.2
-  // against 3.0 ms; FP64 128^3 4.0 against 4.3 ms).  FP64 512^3 solve with
-  // 64 x 32 tiles in XCD-aware order: 45.4 against 47.5 ms with 64 x 16.
-  // FP32 levels of 128 rows whose width is a multiple of 128 (whole tiles)
-  // take 128 x 32 too (smoother at 128^3: 13.3 against 17.5 us; at 96^3 and
-  // 192^3, with partial tiles, 64 x 8 stays faster: 10.5 against 12.4 us
-  // and 26.7 against 31.4 us).
+  // Unless set, the tile follows the level: 64 x 32 (FP64) and 128 x 32 (FP32)
+  // on levels of 256 rows or more (FP64 512^3 solve with 64 x 32 tiles in
+  // XCD-aware order: 45.4 against 47.5 ms with 64 x 16).  FP32 levels of 128
+  // rows whose width is a multiple of 128 (whole tiles) take 128 x 32 too
+  // (13.3 against 17.5 us an iteration at 128^3; with partial tiles, 192^3,
+  // 64 x 8 stays faster: 26.7 against 31.4 us).  Otherwise 64 x 8, whose
+  // smaller blocks keep more CUs busy, but for FP64 levels where 64 x 32
+  // tiles make exactly one wave of blocks and their rows are three quarters
+  // full or more: solves at 128^3 2.41 against 2.46 ms, 512 x 32 x 256 2.52
+  // against 2.61, 64 x 48 x 1024 2.91 against 2.95, 96 x 240 x 96 3.20
+  // against 3.34.  Outside that 64 x 8 is the faster: 144^3 4.23 against
+  // 4.86, 160^3 3.72 against 4.05, 192^3 4.38 against 4.69; 1024 x 16 x 128,
+  // whose rows fill half of a tile, 1.92 against 1.97.
   static bool big_level(const DevLevel<T>& d) {
-    return d.ny >= 256 || (sizeof(T) == 4 && d.ny >= 128 && d.nx % 128 == 0);
+    if (d.ny >= 256 || (sizeof(T) == 4 && d.ny >= 128 && d.nx % 128 == 0)) return true;
+    const long gy = (d.ny + 31) / 32;
+    return sizeof(T) == 8 && 4L * d.ny >= 3 * 32 * gy &&
+           one_wave(d, (long)((d.nx + FTX - 1) / FTX) * gy, fused_resident<FTX, 32, 1>());
   }
   static int default_tx(const DevLevel<T>& d) { return (sizeof(T) == 4 && big_level(d)) ? FTX : 64; }
   static int default_ty(const DevLevel<T>& d) { return big_level(d) ? 32 : 8; }
