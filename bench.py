@@ -850,9 +850,11 @@ def main():
             "traffic_write": round(tr["WRITE_SIZE"]) if tr else None,
             "kernel": kname64, "kernel_down": kname64.replace("k_rb_fused<", "k_rb_fused_down<"),
             "avg_ms": avg64, "launches": n64, "bytes_per_launch": nbytes64,
-            "timing": f"HIP events on the solve stream around every plain iteration on the {n}^3 level inside "
-                      f"{ev_steps} FP64 solves run after the timed ones (both kernels: a plain iteration that "
-                      "follows an upward launch on the level marches down)",
+            "iterations_per_launch": 2 if kname64.startswith("k_sweep") else 1,
+            "timing": f"HIP events on the solve stream around every plain launch on the {n}^3 level inside "
+                      f"{ev_steps} FP64 solves run after the timed ones (k_sweep: two iterations a launch; "
+                      "k_rb_fused: one, downward where it follows an upward one); bytes_per_launch is one "
+                      "pass, x and b read and x written",
             "stream_ceiling_gbs": round(stream_gbs, 1), "frac_of_stream_ceiling": round(achieved / stream_gbs, 4),
             "back_to_back": {"avg_ms": bb64, "frac": frac(nbytes64, bb64),
                              "note": f"{a.smoother_reps} launches in a row after {a.smoother_reps} untimed ones "
@@ -860,6 +862,7 @@ def main():
     roof32 = {"achieved": round(achieved32, 1), "frac": round(achieved32 / HBM_PEAK_GBS, 4), "kernel": kname32,
               "kernel_down": kname32.replace("k_rb_fused<", "k_rb_fused_down<"),
               "avg_ms": avg32, "launches": n32, "bytes_per_launch": nbytes32,
+              "iterations_per_launch": 2 if kname32.startswith("k_sweep") else 1,
               "timing": f"HIP events around every launch on the {n}^3 level inside {ev_steps} mixed solves "
                         "(default options) run after the timed ones",
               "back_to_back": {"avg_ms": bb32, "frac": frac(nbytes32, bb32)}}
