@@ -340,7 +340,8 @@ int pepsmg_ctx::alloc_scratch() {
   HIP_TRY(hipEventCreate(&ev1));
   HIP_TRY(hipEventCreateWithFlags(&ev_norm, hipEventDisableTiming));
   HIP_TRY(hipEventCreateWithFlags(&ev_entry, hipEventDisableTiming));
-  HIP_TRY(hipHostMalloc((void**)&h_scalars, 8 * sizeof(double), hipHostMallocDefault));
+  HIP_TRY(hipHostMalloc((void**)&h_scalars, 8 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
+  HIP_TRY(hipHostGetDevicePointer((void**)&hd_scalars, h_scalars, 0));
   return PEPSMG_OK;
 }
 
@@ -367,7 +368,7 @@ void pepsmg_ctx::release() {
     if (e) hipEventDestroy(e);
   timer.ev.clear();
   if (h_scalars) hipHostFree(h_scalars);
-  h_scalars = nullptr;
+  h_scalars = hd_scalars = nullptr;
   if (stream) hipStreamDestroy(stream);
   stream = nullptr;
 }
@@ -606,7 +607,6 @@ static int solve_fp64(pepsmg_ctx* c, int nu, double tol, double omega, pepsmg_st
     if (rc) return rc;
   }
   DevLevel<double>& f = h.lv[0];
-  double hs[2];
   // With the fused RBGS smoother the convergence norm of a cycle's result
   // (:1970-1971) comes out of the first pre-smoothing iteration of the next
   // cycle, which evaluates |b - A x|^2 of the x it starts from while it
@@ -624,10 +624,9 @@ static int solve_fp64(pepsmg_ctx* c, int nu, double tol, double omega, pepsmg_st
   double rho = 1.0;
   int first = 1;   // first cycle to run
   if (!fold) {
-    op.resid_norm_march(f, f.x, f.b, nullptr, c->d_partial, c->d_scalars + 0);  // :1924-1925
-    HIP_TRY(hipMemcpyAsync(hs, c->d_scalars, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    op.resid_norm_march(f, f.x, f.b, nullptr, c->d_partial, c->hd_scalars + 0);  // :1924-1925
     HIP_TRY(hipStreamSynchronize(c->stream));
-    res0 = hs[0];
+    res0 = c->h_scalars[0];
     int rc = check_res0(res0);
     if (rc) return rc;
     if (res0 == 0.0) {   // x0 is exact: no cycle
@@ -682,9 +681,8 @@ static int solve_fp64(pepsmg_ctx* c, int nu, double tol, double omega, pepsmg_st
         op.fused_iter(f, omega, (cyc == 1 && direct) ? 3 : 2, c->d_partial);
       }
       hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, c->stream, c->d_partial, nbc,
-                         c->d_scalars + (cyc == 1 ? 0 : 1));
+                         c->hd_scalars + (cyc == 1 ? 0 : 1));
       if (cyc > 1) {
-        HIP_TRY(hipMemcpyAsync(c->h_scalars, c->d_scalars, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(hipEventRecord(c->ev_norm, c->stream));
         // While the host waits for the norm, the GPU runs the second
         // iteration into the spare buffer f.r (or, when both iterations are
@@ -721,11 +719,10 @@ static int solve_fp64(pepsmg_ctx* c, int nu, double tol, double omega, pepsmg_st
     smooth_level(c, op, h, cg, 0, nu, omega, false, true, dual ? 4 : 0);  // :1965-1967
     if (!fold || cyc == c->ncycle) {
       c->sol_out_done = dual_cycle == cyc;
-      op.resid_norm_march(f, f.x, f.b, nullptr, c->d_partial, c->d_scalars + 1);  // :1970-1971
-      HIP_TRY(hipMemcpyAsync(hs, c->d_scalars, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+      op.resid_norm_march(f, f.x, f.b, nullptr, c->d_partial, c->hd_scalars + 1);  // :1970-1971
       HIP_TRY(hipStreamSynchronize(c->stream));
-      if (fold) res0 = hs[0];
-      int stop = check(cyc, hs[1]);
+      if (fold) res0 = c->h_scalars[0];
+      int stop = check(cyc, c->h_scalars[1]);
       if (stop < 0) return stop;
       if (stop) break;
     }
@@ -793,7 +790,7 @@ static int solve_mixed(pepsmg_ctx* c, int nu, double tol, double omega, std::vec
     else
       hipLaunchKernelGGL((k_refine_start<RESID_TY>), dim3((unsigned)nb), dim3(MARCH_THREADS), 0, c->stream, ux + uo,
                          ub + uo, f32.b, f.L(), U, G, c->d_partial);
-    hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, c->stream, c->d_partial, nb, c->d_scalars);
+    hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, c->stream, c->d_partial, nb, c->hd_scalars);
     x_caller = true;
     c->sol_out_done = true;
   };
@@ -818,7 +815,7 @@ static int solve_mixed(pepsmg_ctx* c, int nu, double tol, double omega, std::vec
         hipLaunchKernelGGL((k_refine_step<RESID_TY>), dim3((unsigned)nb), dim3(MARCH_THREADS), 0, c->stream, xs,
                            f32.x, bsrc, f32.b, f.x2, f.L(), LX, LB, G, c->d_partial);
     }
-    hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, c->stream, c->d_partial, nb, c->d_scalars);
+    hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, c->stream, c->d_partial, nb, c->hd_scalars);
     if (!last) {
       std::swap(f.x, f.x2);
       x_caller = false;
@@ -845,7 +842,6 @@ static int solve_mixed(pepsmg_ctx* c, int nu, double tol, double omega, std::vec
   // the read-back leaves no gap; skipped when the step is predicted to stop.
   bool ahead = false;
   auto read_norm = [&](bool run_ahead) -> int {
-    HIP_TRY(hipMemcpyAsync(c->h_scalars, c->d_scalars, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipEventRecord(c->ev_norm, c->stream));
     ahead = run_ahead;
     if (ahead) smooth_level(c, op, g, cg, 0, nui, om, true, false);
@@ -1073,20 +1069,22 @@ int pepsmg_multigrid_solve_vcycle_device(pepsmg_ctx* c, double* d_sol, double* d
   // (with the same check).
   const bool direct = c->opt.precision == 1 || (c->opt.fused_smoother && c->opt.smoother == 0 && maxiteration > 0 &&
                                                 c->ncycle > 0);
-  hipMemsetAsync(c->d_flag, 0, sizeof(int), c->stream);
+  // (the flag is there with the solve's first norm: the solve never reads
+  // ghost cells and writes nothing of the caller's before the check)
+  int* h_flag = c->ghost_flag_host();
+  *h_flag = 0;
+  hipError_t e = hipSuccess;
   if (direct) {
     const long items = 2L * (f.nx + 2) * (f.ny + 2) + 2L * f.nz * (f.nx + 2) + (long)f.ny * f.nz;
     const unsigned nb = (unsigned)std::min<long>((items + 255) / 256, 2048);
-    hipLaunchKernelGGL(k_ghost_check, dim3(nb), dim3(256), 0, c->stream, d_sol, f.nx, f.ny, f.nz, c->d_flag);
+    hipLaunchKernelGGL(k_ghost_check, dim3(nb), dim3(256), 0, c->stream, d_sol, f.nx, f.ny, f.nz,
+                       c->ghost_flag_dev());
   } else {
+    hipMemsetAsync(c->d_flag, 0, sizeof(int), c->stream);
     pack(c->stream, f.x, d_sol, f, c->d_flag);
     pack(c->stream, f.b, d_rhs, f, (int*)nullptr);
+    e = hipMemcpyAsync(h_flag, c->d_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream);
   }
-  // the flag is read back with the solve's first norm (the solve never
-  // reads ghost cells and writes nothing of the caller's before the check)
-  int* h_flag = c->ghost_flag_host();
-  *h_flag = 0;
-  hipError_t e = hipMemcpyAsync(h_flag, c->d_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream);
   if (e != hipSuccess) rc = hip_fail(e, "pack");
   if (!rc) rc = run_solve(c, maxiteration, tolerance, omega_sor, st, direct ? d_sol : nullptr, direct ? d_rhs : nullptr);
   if (rc) {
