@@ -1,6 +1,7 @@
 // pepsmg_block.h -- NIT red/black iterations on small levels in one launch
 // (gfx950): from x, from x = 0 or from x plus the prolongation of the coarser
-// level, out of place.
+// level, out of place; REST: then the residual restricted into the coarser
+// level's b.
 //
 // Bound: latency.  On levels of 128^3 cells and fewer a z-march waits for a
 // memory round trip at each of its few plane steps (k_rb_fused takes 6 to 8
@@ -33,6 +34,8 @@ struct BlockArgs {
   T omega;
   int gx, gy;                // tiles along x and y
   double* partial;           // NORM: per-block sums of (b - A x_in)^2
+  T* bc;                     // REST: the coarser level's b (C and RW: its layout and the weights)
+  RestrictW<T> RW;
   T* ext;                    // FP64: the caller's array that also receives x_out (layout U), or null
   Lvl<T> U;
 };
@@ -48,10 +51,11 @@ using BlockLarge = BlockTile<32, 8, 8, 1024>;
 // what that gains: the half-sweeps are short of instruction slots.)
 using BlockTall = BlockTile<32, 16, 8, 1024>;
 
-template <typename T, typename B, int NIT, int PRE>
+template <typename T, typename B, int NIT, int PRE, bool REST = false>
 struct BlockShape {
-  static constexpr int H = 2 * NIT;
-  static constexpr int PX = (B::BX + 2 * H) / 2, RY = B::BY + 2 * H, RZ = B::BZ + 2 * H;
+  // ring along y and z, and along x (even, so that pairs keep their parity)
+  static constexpr int H = 2 * NIT + (REST ? 1 : 0), HX = 2 * NIT + (REST ? 2 : 0);
+  static constexpr int PX = (B::BX + 2 * HX) / 2, RY = B::BY + 2 * H, RZ = B::BZ + 2 * H;
   static constexpr int NPAIR = PX * RY * RZ, PP = (NPAIR + B::NT - 1) / B::NT;
   // coarse cells the region interpolates from
   static constexpr int CX = PX + 2, CY = RY / 2 + 2, CZ = RZ / 2 + 2, NC = CX * CY * CZ;
@@ -61,12 +65,12 @@ struct BlockShape {
 };
 
 // tile `bid` of the level
-template <typename T, typename B, int NIT, int PRE, bool NORM>
+template <typename T, typename B, int NIT, int PRE, bool NORM, bool REST = false>
 __device__ __forceinline__ void block_tile(const BlockArgs<T>& A, int bid) {
-  using S = BlockShape<T, B, NIT, PRE>;
+  using S = BlockShape<T, B, NIT, PRE, REST>;
   using V2 = typename SwPair<T>::type;
   constexpr bool F64 = sizeof(T) == 8;
-  constexpr int H = S::H, PX = S::PX, RY = S::RY, RZ = S::RZ, NP = S::NPAIR, PP = S::PP, NT = B::NT;
+  constexpr int H = S::H, HX = S::HX, PX = S::PX, RY = S::RY, RZ = S::RZ, NP = S::NPAIR, PP = S::PP, NT = B::NT;
   extern __shared__ __align__(16) unsigned char bl_smem[];
   T* const xs = reinterpret_cast<T*>(bl_smem);       // first cells of the pairs, then the second ones
   T* const cx = xs + 2 * NP;                         // cwx, cex of the region's columns (0 outside the level)
@@ -78,7 +82,7 @@ __device__ __forceinline__ void block_tile(const BlockArgs<T>& A, int bid) {
   const Lvl<T>& L = A.L;
   const int t = threadIdx.x;
   const int bx = bid % A.gx, byz = bid / A.gx;
-  const int i0 = 1 + bx * B::BX - H, j0 = 1 + (byz % A.gy) * B::BY - H, k0 = 1 + (byz / A.gy) * B::BZ - H;   // i0 odd
+  const int i0 = 1 + bx * B::BX - HX, j0 = 1 + (byz % A.gy) * B::BY - H, k0 = 1 + (byz / A.gy) * B::BZ - H;   // i0 odd
 
   // ---- all loads ----
   V2 xv[PP], bv[PP];
@@ -99,7 +103,7 @@ __device__ __forceinline__ void block_tile(const BlockArgs<T>& A, int bid) {
     dist[p][0] = v0 ? min(dyz, min(2 * px, 2 * PX - 1 - 2 * px)) : -1;
     dist[p][1] = v1 ? min(dyz, min(2 * px + 1, 2 * PX - 2 - 2 * px)) : -1;
     first[p] = ((j + k) & 1) == 0;
-    tile[p] = v0 && px >= H / 2 && px < PX - H / 2 && ry >= H && ry < RY - H && rz >= H && rz < RZ - H;
+    tile[p] = v0 && px >= HX / 2 && px < PX - HX / 2 && ry >= H && ry < RY - H && rz >= H && rz < RZ - H;
     // an odd column <= nx keeps the pair inside the padded row
     const int ic = v0 ? i : 1, jc = min(max(j, 1), L.ny), kc = min(max(k, 1), L.nz);
     const long g = lidx(L, ic, jc, kc);
@@ -136,6 +140,17 @@ __device__ __forceinline__ void block_tile(const BlockArgs<T>& A, int bid) {
       pw[2 * t] = g & 1 ? p[g] : m[g];
       pw[2 * t + 1] = g & 1 ? p[g + 1] : m[g - 1];
     }
+  }
+  // REST: the thread's coarse cell and its weights
+  constexpr int QX = B::BX / 2, QY = B::BY / 2, QZ = B::BZ / 2;
+  const int qx = t % QX, qy = t / QX % QY, qz = t / (QX * QY);
+  const int ic = bx * QX + qx + 1, jc = (byz % A.gy) * QY + qy + 1, kc = (byz / A.gy) * QZ + qz + 1;
+  const bool rest = REST && t < QX * QY * QZ && ic <= A.C.nx && jc <= A.C.ny && kc <= A.C.nz;
+  T ax1 = T(0), ax2 = T(0), ay1 = T(0), ay2 = T(0), az1 = T(0), az2 = T(0);
+  if (REST && rest) {
+    ax1 = A.RW.wx[2 * ic - 1], ax2 = A.RW.wx[2 * ic];
+    ay1 = A.RW.wy[2 * jc - 1], ay2 = A.RW.wy[2 * jc];
+    az1 = A.RW.wz[2 * kc - 1], az2 = A.RW.wz[2 * kc];
   }
   if constexpr (PRE == SW_PROLONG) {
     // coarse region: the parents of the fine region and one cell around
@@ -260,11 +275,55 @@ __device__ __forceinline__ void block_tile(const BlockArgs<T>& A, int bid) {
       else u[0] = o.x;
     }
   }
+  if constexpr (REST) {
+    // the residual of the tile (the last half-sweep also covered one cell
+    // around it), in place of x, and the restriction from there
+    // (restrict_axis's weights, k_restrict's terms and order)
+    static_assert(QX * QY * QZ <= NT, "a coarse cell per thread");
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < PP; p++) {
+      if (!tile[p]) continue;
+      const T *ky = cy + 2 * (at[p] >> 8 & 255), *kz = cz + 2 * (at[p] >> 16);
+      const T c3 = ky[0], c4 = ky[1], c5 = kz[0], c6 = kz[1];
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        const T* kx = cx + 2 * (2 * (at[p] & 255) + c);
+        const T c0 = diag(kx[0], kx[1], c3, c4, c5, c6);
+        const T* o = xs + c * NP + id[p];
+        const T* w = xs + (1 - c) * NP + id[p] - (1 - c);
+        const T ax = c0 * o[0] + kx[0] * w[0] + kx[1] * w[1] + c3 * o[-PX] + c4 * o[PX] + c5 * o[-PX * RY] +
+                     c6 * o[PX * RY];
+        if (c) bv[p].y = bv[p].y - ax;
+        else bv[p].x = bv[p].x - ax;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < PP; p++) {
+      if (!tile[p]) continue;
+      xs[id[p]] = bv[p].x;
+      xs[NP + id[p]] = bv[p].y;
+    }
+    __syncthreads();
+    if (rest) {
+      const T v111 = ax1 * ay1 * az1, v211 = ax2 * ay1 * az1, v121 = ax1 * ay2 * az1, v221 = ax2 * ay2 * az1;
+      const T v112 = ax1 * ay1 * az2, v212 = ax2 * ay1 * az2, v122 = ax1 * ay2 * az2, v222 = ax2 * ay2 * az2;
+      const T vol = v111 + v211 + v121 + v221 + v112 + v212 + v122 + v222;
+      // z, p: the odd and the even child along an axis
+      auto R = [&](int a, int bb, int cc) {
+        return xs[a * NP + ((H + 2 * qz + cc) * RY + H + 2 * qy + bb) * PX + HX / 2 + qx];
+      };
+      const T sum = v111 * R(1, 1, 1) + v211 * R(0, 1, 1) + v121 * R(1, 0, 1) + v221 * R(0, 0, 1) +
+                    v112 * R(1, 1, 0) + v212 * R(0, 1, 0) + v122 * R(1, 0, 0) + v222 * R(0, 0, 0);
+      A.bc[lidx(A.C, ic, jc, kc)] = sum / vol;
+    }
+  }
 }
 
-template <typename T, typename B, int NIT, int PRE, bool NORM>
+template <typename T, typename B, int NIT, int PRE, bool NORM, bool REST>
 __global__ void __launch_bounds__(B::NT) k_block(BlockArgs<T> A) {
-  block_tile<T, B, NIT, PRE, NORM>(A, blockIdx.x);
+  block_tile<T, B, NIT, PRE, NORM, REST>(A, blockIdx.x);
 }
 
 }  // namespace pepsmg

@@ -423,6 +423,21 @@ static void smooth_level(pepsmg_ctx* c, Ops<T>& op, Hier<T>& h, CgBufs<T>* cg, i
   op.rbgs(d, d.x, d.b, nu, omega, zero_start);
 }
 
+// nu pre-smoothing iterations on level l and the restriction of the residual
+// into level l + 1's b (src/multigrid.f90:1931-1933, :1938-1941), in one
+// launch where the level allows it
+template <typename T>
+static void smooth_restrict(pepsmg_ctx* c, Ops<T>& op, Hier<T>& h, CgBufs<T>* cg, int l, int nu, T omega,
+                            bool zero_start) {
+  DevLevel<T>& d = h.lv[l];
+  if (c->opt.fused_smoother && c->opt.smoother == 0 && nu > 0 && op.blocks(d) && op.restricts(d, h.lv[l + 1])) {
+    op.iterate_restrict(d, omega, nu, zero_start, &h.lv[l + 1]);
+    return;
+  }
+  smooth_level(c, op, h, cg, l, nu, omega, zero_start, false);
+  op.residual_restrict(d, h.lv[l + 1], d.x, d.b);
+}
+
 // Coarsest level: FP64 solve in one workgroup (src/multigrid.f90:1944-1949,
 // tolerance = the V-cycle tolerance, at most 1000 iterations).
 static void coarse_solve64(pepsmg_ctx* c, DevLevel<double>& d, double omega, double tol, int* slot) {
@@ -548,9 +563,7 @@ static void vcycle_coarse_part(pepsmg_ctx* c, Ops<T>& op, Hier<T>& h, CgBufs<T>*
   if constexpr (std::is_same<T, float>::value) A.cinv = c->d_cinv;   // exact coarsest solve (inner cycles)
   int last = std::min(s, L) - 1;   // last level of the per-level down-leg
   for (int l = 1; l <= last; l++) {
-    DevLevel<T>& d = h.lv[l];
-    smooth_level(c, op, h, cg, l, nu, omega, true, false);
-    op.residual_restrict(d, h.lv[l + 1], d.x, d.b);
+    smooth_restrict(c, op, h, cg, l, nu, omega, true);
   }
   if (s <= L) {
     A.gxs = h.lv[s].x;   // current buffers
@@ -838,13 +851,13 @@ static int solve_mixed(pepsmg_ctx* c, int nu, double tol, double omega, std::vec
   const int nui = c->opt.inner_nu > 0 ? c->opt.inner_nu : nu;
   const int nup = c->opt.inner_nu_post > 0 ? c->opt.inner_nu_post : nui;
   // The host reads each norm while the GPU already runs the next step's
-  // first pre-smoothing (it needs only r32, and touches no FP64 array), so
+  // first pre-smoothing and restriction (which need only r32, and touch no FP64 array), so
   // the read-back leaves no gap; skipped when the step is predicted to stop.
   bool ahead = false;
   auto read_norm = [&](bool run_ahead) -> int {
     HIP_TRY(hipEventRecord(c->ev_norm, c->stream));
     ahead = run_ahead;
-    if (ahead) smooth_level(c, op, g, cg, 0, nui, om, true, false);
+    if (ahead) smooth_restrict(c, op, g, cg, 0, nui, om, true);
     HIP_TRY(hipEventSynchronize(c->ev_norm));
     return PEPSMG_OK;
   };
@@ -877,8 +890,7 @@ static int solve_mixed(pepsmg_ctx* c, int nu, double tol, double omega, std::vec
     double rho_prev = rho;
     for (int q = 0; q < nin; q++) {
       int* slot = (ncyc < c->citers_cap) ? c->d_citers + ncyc : nullptr;
-      if (!(q == 0 && ahead)) smooth_level(c, op, g, cg, 0, nui, om, q == 0, false);
-      op.residual_restrict(f32, g.lv[1], f32.x, f32.b);
+      if (!(q == 0 && ahead)) smooth_restrict(c, op, g, cg, 0, nui, om, q == 0);
       vcycle_coarse_part<float>(c, op, g, cg, nui, nup, om, tol, slot);
       smooth_level(c, op, g, cg, 0, nup, om, false, true);
       ncyc++;

@@ -73,3 +73,25 @@ def test_fp32_tall_tiles(dims, omega, nu):
     rbgs_iterator_fp32(x, b, sdm_from(g), nu, omega)
     O.rbgs_iterator(xo, A, b, nu, omega)
     assert np.abs(x - xo).max() <= 1e-6 * (1 + nu) * np.abs(xo).max()
+
+
+@pytest.mark.parametrize("dims,nlevel", [((48, 24, 40), 3), ((144, 40, 24), 3), ((80, 72, 88), 3)])
+@pytest.mark.parametrize("nu", [1, 2, 3, 4])
+def test_restricting_blocks_bitwise(dims, nlevel, nu):
+    """Per-level solves down to the coarsest level, whose pre-smoothing launches also restrict: partial tiles on
+    every axis, the last launch of one or two iterations, from 0 and from x."""
+    import torch
+    g = O.Grid(*dims, l=tuple(d / 16 for d in dims), a=(1.0, 1.02, 1.01))
+    A = g.matrix()
+    b = O.uniform_field(*dims, 26)
+    mo = O.Multigrid(g, nlevel, 4)
+    xo, ro = O.padded(*dims), O.padded(*dims)
+    nc, hist, cit, res0 = mo.solve_vcycle(xo, ro, A, b, nu, 1e-9, 1.0)
+    mg = Multigrid(sdm_from(g), nlevel, 4, coarse_switch=0)
+    d_b = torch.from_numpy(b).cuda()
+    d_x = torch.zeros_like(d_b)
+    res = mg.solve_vcycle_device(d_x.data_ptr(), 0, d_b.data_ptr(), nu, 1e-9, 1.0)
+    torch.cuda.synchronize()
+    assert res.cycles == nc
+    assert np.max(np.abs(res.history - hist)) <= 1e-12
+    assert np.array_equal(d_x.cpu().numpy(), xo)
