@@ -274,6 +274,10 @@ static void cg_iterate(Ops<T>& op, DevLevel<T>& d, T* x, const T* b, T* r, T* p,
   if (zero_x) {
     hipLaunchKernelGGL((k_cg_start0<T>), dim3(eb), eblk, 0, op.s, r, p, b, d.L(), prr[0]);
     rr[0] = {prr[0], eb};
+    if (!march) {   // k_cg_p reads the scalar
+      hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, op.s, prr[0], eb, sc + 0);
+      rr[0] = {sc + 0, 1};
+    }
   } else if (march) {
     hipLaunchKernelGGL((k_resid_march<T, RESID_TY, 4>), dim3(mb), dim3(MARCH_THREADS), 0, op.s, x, (const float*)nullptr,
                        b, r, (float*)nullptr, p, d.L(), G, prr[0]);

@@ -1,0 +1,36 @@
+"""CG iterations on levels whose march has more blocks than the reductions hold partial sums: they run the separate
+mat-vec, dot product and direction update."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from peps_mg_amd import geometry
+from peps_mg_amd.multigrid import Multigrid
+
+pytestmark = pytest.mark.gpu
+
+
+def sdm_from(g):
+    return geometry.Subdomain(g.nx, g.ny, g.nz, 0, 0, 0, g.sox, g.soy, g.soz, g.dxm, g.dym, g.dzm, g.dxg, g.dyg,
+                              g.dzg, g.xg, g.yg, g.zg)
+
+
+@pytest.mark.parametrize("ny", [1100000, 4300000])
+def test_start_from_zero(ny):
+    """One inner cycle of a mixed solve, whose finest level starts from x = 0, is the oracle's first CG(4) V-cycle
+    from x = 0 but for its rounding: nine CG steps' worth of the FP32 smoothers' bound, 1e-6 each, for the
+    solution (relative to its maximum) and for the residual (relative to the right-hand side: on a level two cells
+    wide and deep, whose matrix has a condition number below 10, it shares the solution's relative error)."""
+    dims = (2, ny, 2)
+    g = O.Grid(*dims, l=tuple(float(d) for d in dims))
+    b = O.uniform_field(*dims, 44)
+    mo = O.Multigrid(g, 2, 1, smoother=1)
+    xo, ro = O.padded(*dims), O.padded(*dims)
+    _, hist, _, _ = mo.solve_vcycle(xo, ro, g.matrix(), b, 4, 1e-12, 1.0)
+    mg = Multigrid(sdm_from(g), 2, 1, smoother=1, precision=1, inner_cycles=1, inner_nu=4, inner_nu_post=4)
+    x, r = O.padded(*dims), O.padded(*dims)
+    res = mg.solve_vcycle(x, r, None, b, 4, 1e-12, 1.0)
+    mg.destroy()
+    assert res.cycles == 1
+    assert np.abs(x - xo).max() <= 9e-6 * np.abs(xo).max()
+    assert abs(res.rho - hist[0]) <= 9e-5, (res.rho, hist[0])
