@@ -362,6 +362,7 @@ struct PartialSum {
 // formed side by side (sh: 2 RED_THREADS / 64 doubles).
 __device__ __forceinline__ double partial_ratio(const PartialSum& num, const PartialSum& den, double* sh) {
   constexpr int NW = RED_THREADS / 64;
+  if (num.n == 1 && den.n == 1) return num.p[0] / den.p[0];
   double a = 0.0, d = 0.0;
   const int n = max(num.n, den.n);
   for (int c = threadIdx.x; c < n; c += RED_THREADS) {

@@ -26,9 +26,10 @@ namespace pepsmg {
 // last iteration it is not needed: p is local to the reference routine).
 // Scalars stay on the device, (r, r) at the start of an iteration (temp1) and
 // (Ap, p) (temp2) as their partial sums, which the kernels that need them add
-// up (partial_ratio); alpha and beta are formed in FP64 by every thread as the
-// reference does (:209, :223).  A 128^3 CG(4) solve ran 638 reductions of one
-// block and 3.4 us each between its kernels: 7.5 ms with them, 6.6 ms without.
+// up (partial_ratio) on all but the largest levels (CG_FOLD); alpha and beta
+// are formed in FP64 by every thread as the reference does (:209, :223).  A
+// 128^3 CG(4) solve ran 638 reductions of one block and 3.4 us each between
+// its kernels: 7.5 ms with them, 6.6 ms without.
 constexpr int CG_WAVES = 4;
 
 // rows (j, k) of a level dealt to waves; each lane handles pairs (i odd, i+1)
@@ -263,25 +264,35 @@ static void cg_iterate(Ops<T>& op, DevLevel<T>& d, T* x, const T* b, T* r, T* p,
   const dim3 eblk(64 * CG_WAVES);
   MarchGrid G = Ops<T>::march_grid(d, RESID_TY, false);
   const int mb = G.gx * G.gy * G.nch;
-  // partial sums of (Ap, p) and, by turns, of (r, r)
-  constexpr int CAP = PARTIAL_CAP / 4;
-  const bool march = mb <= CAP;
-  static_assert(RED_BLOCKS <= CAP, "partial sums");
+  const bool march = mb <= PARTIAL_CAP;
+  // Every block that needs a scalar adds up its partial sums itself on levels
+  // of up to CG_FOLD of them.  Beyond, that reading grows with the square of
+  // the blocks, and one block adds them up in between.  Two CG(4) cycles by
+  // folding and with the separate sums: 512 x 512 x 64 (2048 sums) FP64 6.65
+  // against 7.2 ms, mixed 2.49 against 2.74; 1024 x 512 x 64 (4096) 12.2
+  // against 12.8 and 4.47 against 4.65; 2048 x 1024 x 64 (16384) 47.0 against
+  // 47.3 and 16.1 against 15.9; 4096 x 2048 x 64 (65536) 193 against 177 and
+  // 66.2 against 56.4.
+  constexpr int CG_FOLD = 4096;
+  static_assert(RED_BLOCKS <= CG_FOLD && 3 * CG_FOLD <= PARTIAL_CAP, "partial sums");
+  const bool fold = mb <= CG_FOLD;
+  // partial sums of (Ap, p) and, by turns, of (r, r); without folding each is used up at once
   double* pap = partial;
-  double* prr[2] = {partial + CAP, partial + 2 * CAP};
+  double* prr[2] = {partial + (fold ? CG_FOLD : 0), partial + (fold ? 2 * CG_FOLD : 0)};
+  auto sum = [&](const double* p, int n, int slot) -> PartialSum {
+    if (fold) return {p, n};
+    hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, op.s, p, n, sc + slot);
+    return {sc + slot, 1};
+  };
   PartialSum rr[2], ap2;
   // start: r = b - A x, p = r, temp1 = (r, r)  (:196-204)
   if (zero_x) {
     hipLaunchKernelGGL((k_cg_start0<T>), dim3(eb), eblk, 0, op.s, r, p, b, d.L(), prr[0]);
-    rr[0] = {prr[0], eb};
-    if (!march) {   // k_cg_p reads the scalar
-      hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, op.s, prr[0], eb, sc + 0);
-      rr[0] = {sc + 0, 1};
-    }
+    rr[0] = sum(prr[0], eb, 0);
   } else if (march) {
     hipLaunchKernelGGL((k_resid_march<T, RESID_TY, 4>), dim3(mb), dim3(MARCH_THREADS), 0, op.s, x, (const float*)nullptr,
                        b, r, (float*)nullptr, p, d.L(), G, prr[0]);
-    rr[0] = {prr[0], mb};
+    rr[0] = sum(prr[0], mb, 0);
   } else {
     op.resid_norm(d, x, b, r, partial, sc + 0);
     hipMemcpyAsync(p, r, d.ncell * sizeof(T), hipMemcpyDeviceToDevice, op.s);
@@ -296,12 +307,12 @@ static void cg_iterate(Ops<T>& op, DevLevel<T>& d, T* x, const T* b, T* r, T* p,
     if (march && it > 0) {   // p = r + beta p (:223-229) folded into A p (:206-207)
       hipLaunchKernelGGL((k_cg_ap_fold<T, RESID_TY>), dim3(mb), dim3(MARCH_THREADS), 0, op.s, r, p, p2, ap, d.L(),
                          G, pap, rr[cur], rr[nxt]);
-      ap2 = {pap, mb};
+      ap2 = sum(pap, mb, 2);
       std::swap(p, p2);
     } else if (march) {                                             // :206-207
       hipLaunchKernelGGL((k_resid_march<T, RESID_TY, 3>), dim3(mb), dim3(MARCH_THREADS), 0, op.s, p,
                          (const float*)nullptr, (const T*)nullptr, ap, (float*)nullptr, (T*)nullptr, d.L(), G, pap);
-      ap2 = {pap, mb};
+      ap2 = sum(pap, mb, 2);
     } else {
       op.apply(d, ap, p);
       op.dot(d, ap, p, partial, sc + 2);
@@ -309,12 +320,9 @@ static void cg_iterate(Ops<T>& op, DevLevel<T>& d, T* x, const T* b, T* r, T* p,
     }
     hipLaunchKernelGGL((k_cg_xr<T>), dim3(eb), eblk, 0, op.s, x, r, p, ap, rr[cur], ap2, d.L(), zero_x && it == 0,
                        prr[nxt]);                                   // partial (r, r) (:221)
-    rr[nxt] = {prr[nxt], eb};
-    if (!march && it + 1 < nu) {
-      hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, op.s, prr[nxt], eb, sc + nxt);
-      rr[nxt] = {sc + nxt, 1};
+    rr[nxt] = sum(prr[nxt], eb, nxt);
+    if (!march && it + 1 < nu)
       hipLaunchKernelGGL((k_cg_p<T>), dim3(eb), eblk, 0, op.s, p, r, sc, nxt, cur, d.L());
-    }
   }
 }
 
