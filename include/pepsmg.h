@@ -71,9 +71,10 @@ typedef struct pepsmg_options {
   int32_t tile_y;          /* fused smoother tile height 8, 16 or 32 cells (0: per level, 32 on levels
                               of 256 rows or more and where it fills the device exactly, else 8); blocks
                               have max(256, tile_x * tile_y / 4) threads; 32-row tiles load one plane
-                              ahead.  Tiles and look-ahead apply to single-iteration launches only: levels
-                              smoothed two iterations at a time (large ones in one pass, small ones by
-                              blocks in LDS) have decompositions of their own */
+                              ahead.  With tile_x, tile_y and a look-ahead of two planes all unset, large
+                              levels take two iterations in one pass and small ones two by blocks in LDS,
+                              in decompositions of their own; setting one runs every level one iteration
+                              a launch */
   int32_t verbose;         /* 1: print the reference's [MG] cycle lines */
   int32_t tile_x;          /* FP32 fused smoother tile width 64 or 128 cells (0: 128 on levels of 256
                               rows or more, 64 below); FP64 uses 64 */
@@ -272,8 +273,8 @@ int pepsmg_batch_set_options(pepsmg_batch *batch, const pepsmg_options *opt);
 int32_t pepsmg_batch_size(const pepsmg_batch *batch);
 
 /* Fused-smoother tile shape per problem (arrays of nprob; 0 or NULL: the
- * options' tile_x / tile_y), where a level's items run single-iteration
- * launches.  Items of different shapes run in separate launches; the
+ * options' tile_x / tile_y).  Problems with a tile run one iteration a
+ * launch, the others also two (pepsmg_options).  Items of different shapes run in separate launches; the
  * autotuner picks the shape per grid size. */
 int pepsmg_batch_set_tiles(pepsmg_batch *batch, const int32_t *tile_x, const int32_t *tile_y);
 

@@ -2,16 +2,18 @@
 
 Everything is measured on the GPU through the C-ABI; nothing is modelled:
 
-* ``tune_tiles`` times the fine-level fused smoother of one grid
+* ``tune_tiles`` times the fine-level single-iteration smoother of one grid
   (``pepsmg_bench_smoother``, HIP events) for each tile shape and prefetch
   depth and returns the fastest;
 * ``tune_solver`` times complete solves over a small space of schedule
   options (FP32 V-cycles per refinement step, their pre- and post-smoothing
   steps and SOR factor, size of the levels handed to the persistent coarse
-  kernel) with the tuned tile;
+  kernel), with the tuned tile where a solve is faster with it: a tile that
+  is set takes away the launches of two iterations;
 * ``tune_batch`` gives every problem of a batch the tile tuned for its grid
-  size (one measurement per distinct size) and then picks the schedule
-  options that make the whole batch fastest.
+  size (one measurement per distinct size), or none where the batch is faster
+  without, and then picks the schedule options that make the whole batch
+  fastest.
 
 Results are cached per grid size and precision in a JSON file
 (``$PEPSMG_TUNE_CACHE`` or ``~/.cache/pepsmg_amd/autotune.json``), so a size
@@ -59,8 +61,9 @@ def _key(kind, sdm, precision, extra=""):
 
 
 def tune_tiles(sdm, nlevel, precision, reps=10, use_cache=True):
-    """Fastest (tile_x, tile_y, fused_smoother) for the fine-level smoother
-    of this grid at this precision; returns a dict of option values."""
+    """Fastest (tile_x, tile_y, fused_smoother) for the fine-level
+    single-iteration smoother of this grid at this precision; returns a dict
+    of option values."""
     from .multigrid import Multigrid
     db = _load() if use_cache else {}
     key = _key("tile", sdm, precision)
@@ -76,11 +79,6 @@ def tune_tiles(sdm, nlevel, precision, reps=10, use_cache=True):
         _lib.check(_lib.lib().pepsmg_bench_smoother(mg.h, precision, reps, 1.0, C.byref(avg), C.byref(nb),
                                                     C.byref(kn)))
         timings[f"{tx}x{ty}/pf{pf}"] = avg.value
-        if kn.value.startswith(b"k_sweep"):
-            # this level's smoother takes two iterations a pass and has no tile to choose; the
-            # levels below keep the tile of their size
-            best_ms, best = avg.value, {"tile_x": 0, "tile_y": 0, "fused_smoother": 1}
-            break
         if avg.value < best_ms:
             best_ms, best = avg.value, {"tile_x": tx, "tile_y": ty, "fused_smoother": pf}
     mg.destroy()
@@ -109,9 +107,29 @@ def tune_solver(sdm, nlevel, d_sol, d_rhs, maxiteration=2, tolerance=1e-10, omeg
     if key in db:
         return db[key]
     tiles = _opts(tune_tiles(sdm, nlevel, precision, use_cache=use_cache))
-    mg = Multigrid(sdm, nlevel, 200, precision=precision, **tiles)
+    mg = Multigrid(sdm, nlevel, 200, precision=precision)
     best, best_t, timings = None, float("inf"), {}
     dflt = _lib.default_options()
+
+    def solve_time(repeats):
+        t = float("inf")
+        for _ in range(repeats + 1):
+            d_sol.zero_()
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            r = mg.solve_vcycle_device(d_sol.data_ptr(), 0, d_rhs.data_ptr(), maxiteration, tolerance, omega)
+            torch.cuda.synchronize()
+            if r.converged:
+                t = min(t, time.perf_counter() - t0)
+        return t
+
+    untiled = _opts({k: getattr(dflt, k) for k in tiles})
+    timings["untiled"] = solve_time(max(repeats, 1))
+    mg.set_options(**tiles)
+    timings["tiled"] = solve_time(max(repeats, 1))
+    if timings["untiled"] <= timings["tiled"]:
+        tiles = untiled
+        mg.set_options(**tiles)
     sched = ([(ic, nu, nup, om) for ic in inner_cycles for nu in inner_nu for nup in inner_nu_post
               for om in inner_omega] if precision == 1
              else [(dflt.inner_cycles, dflt.inner_nu, dflt.inner_nu_post, dflt.inner_omega)])
@@ -121,15 +139,7 @@ def tune_solver(sdm, nlevel, d_sol, d_rhs, maxiteration=2, tolerance=1e-10, omeg
                 mg.set_options(coarse_switch=cs, inner_cycles=ic, inner_nu=nui, inner_nu_post=nup, inner_omega=om)
             except _lib.PepsmgError:
                 continue
-            t = float("inf")
-            for _ in range(repeats + 1):
-                d_sol.zero_()
-                torch.cuda.synchronize()
-                t0 = time.perf_counter()
-                r = mg.solve_vcycle_device(d_sol.data_ptr(), 0, d_rhs.data_ptr(), maxiteration, tolerance, omega)
-                torch.cuda.synchronize()
-                if r.converged:
-                    t = min(t, time.perf_counter() - t0)
+            t = solve_time(repeats)
             timings[f"cs{cs}/ic{ic}/nu{nui}-{nup}/om{om}"] = t
             if t < best_t:
                 best_t, best = t, dict(tiles, coarse_switch=cs, inner_cycles=ic, inner_nu=nui, inner_nu_post=nup,
@@ -145,8 +155,9 @@ def tune_solver(sdm, nlevel, d_sol, d_rhs, maxiteration=2, tolerance=1e-10, omeg
 
 def tune_batch(batch, sols, rhss, maxiteration=2, tolerance=1e-10, omega=1.0, inner_cycles=(2, 3),
                inner_nu=(1, 2), inner_nu_post=(1, 2), inner_omega=(1.2, 1.35), repeats=1, use_cache=True):
-    """Per-problem tiles by grid size, then the inner-cycle schedule that
-    makes the whole batch fastest; applies both to `batch` (a BatchSolver)
+    """Per-problem tiles by grid size (0: none set, the faster choice for this
+    batch), then the inner-cycle schedule that makes the whole batch fastest;
+    applies both to `batch` (a BatchSolver)
     and returns {'tiles': {size: tile}, 'inner_cycles': n, 'inner_nu': n,
     'inner_nu_post': n, 'inner_omega': w, 'timings': {...}}."""
     import torch
@@ -160,14 +171,9 @@ def tune_batch(batch, sols, rhss, maxiteration=2, tolerance=1e-10, omega=1.0, in
         t = tiles_by_size[key]
         tx.append(t["tile_x"])
         ty.append(t["tile_y"])
-    batch.set_tiles(tx, ty)
     timings, best, best_t = {}, None, float("inf")
-    o = batch.options
-    sched = ([(ic, nu, nup, om) for ic in inner_cycles for nu in inner_nu for nup in inner_nu_post
-              for om in inner_omega] if precision == 1
-             else [(o.inner_cycles, o.inner_nu, o.inner_nu_post, o.inner_omega)])
-    for ic, nui, nup, om in sched:
-        batch.set_options(inner_cycles=ic, inner_nu=nui, inner_nu_post=nup, inner_omega=om)
+
+    def solve_time(repeats):
         t = float("inf")
         for _ in range(repeats + 1):
             for x in sols:
@@ -178,6 +184,22 @@ def tune_batch(batch, sols, rhss, maxiteration=2, tolerance=1e-10, omega=1.0, in
             torch.cuda.synchronize()
             if all(r.converged for r in res):
                 t = min(t, time.perf_counter() - t0)
+        return t
+
+    batch.set_tiles([0] * len(tx), [0] * len(ty))
+    timings["untiled"] = solve_time(max(repeats, 1))
+    batch.set_tiles(tx, ty)
+    timings["tiled"] = solve_time(max(repeats, 1))
+    if timings["untiled"] <= timings["tiled"]:
+        batch.set_tiles([0] * len(tx), [0] * len(ty))
+        tiles_by_size = {k: {"tile_x": 0, "tile_y": 0} for k in tiles_by_size}
+    o = batch.options
+    sched = ([(ic, nu, nup, om) for ic in inner_cycles for nu in inner_nu for nup in inner_nu_post
+              for om in inner_omega] if precision == 1
+             else [(o.inner_cycles, o.inner_nu, o.inner_nu_post, o.inner_omega)])
+    for ic, nui, nup, om in sched:
+        batch.set_options(inner_cycles=ic, inner_nu=nui, inner_nu_post=nup, inner_omega=om)
+        t = solve_time(repeats)
         timings[f"ic{ic}/nu{nui}-{nup}/om{om}"] = t
         if t < best_t:
             best_t, best = t, (ic, nui, nup, om)

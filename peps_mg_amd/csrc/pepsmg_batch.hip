@@ -502,16 +502,34 @@ static void rec_prolong(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, con
 // FP64, 16 items of 64^3: 3.37 ms without and 3.43 with); the others by blocks
 // up to the same sums as there (the 18 items, no sweeps: 6.2 ms in single
 // iterations, 5.9 with blocks on the coarser levels).  The rest one at a
-// time in the tiles set by the caller; unset, as the single-grid solver, but
-// for levels of 128 rows in FP32: 128 x 32 tiles leave the few blocks of the
-// items that take them alone on the device (two 128^3 items 41 us an
-// iteration; among the 64 x 8 blocks of the others they add 14).
+// time, and so all iterations of an item whose tile the caller set; tiles
+// unset, as the single-grid solver, but for levels of 128 rows in FP32:
+// 128 x 32 tiles leave the few blocks of the items that take them alone on
+// the device (two 128^3 items 41 us an iteration; among the 64 x 8 blocks of
+// the others they add 14).
 template <typename T>
 struct SmoothPlan {
   std::vector<int> sweep, block, fused[2][3];   // fused: by tile width (64, 128) and height (8, 16, 32)
   int shape = 0;                                // block: BlockSmall, BlockLarge (1), BlockTall (2)
   bool prolong_in_block = false;
 };
+
+// item i's tile, 0: not set by the caller (FP64 tiles are 64 wide)
+template <typename T>
+static int set_tile_x(const pepsmg_batch* B, int i) {
+  return sizeof(T) == 8 ? 0 : B->items[i].tile_x ? B->items[i].tile_x : B->opt.tile_x;
+}
+static int set_tile_y(const pepsmg_batch* B, int i) { return B->items[i].tile_y ? B->items[i].tile_y : B->opt.tile_y; }
+
+// adds item i to the groups of single-iteration launches by the tile of its level l
+template <typename T>
+static void add_fused(pepsmg_batch* B, std::vector<Hier<T>*>& H, int l, int i, std::vector<int> (&fused)[2][3]) {
+  int tx = set_tile_x<T>(B, i), ty = set_tile_y(B, i);
+  const bool big = H[i]->lv[l].ny >= 256;
+  if (!tx) tx = big ? Ops<T>::FTX : 64;
+  if (!ty) ty = big ? 32 : 8;
+  fused[sizeof(T) == 4 && tx != 64][ty == 32 ? 2 : ty == 16 ? 1 : 0].push_back(i);
+}
 
 template <typename T>
 static SmoothPlan<T> smooth_plan(pepsmg_batch* B, std::vector<Hier<T>*>& H, int l, int nu) {
@@ -522,7 +540,9 @@ static SmoothPlan<T> smooth_plan(pepsmg_batch* B, std::vector<Hier<T>*>& H, int 
   for (int i = 0; i < B->nitems; i++) {
     if (l >= B->items[i].s) continue;
     const DevLevel<T>& d = H[i]->lv[l];
-    if (nu >= 2 && d.cells() >= 100000 && d.pxy * (long)sizeof(T) <= 0x7fffffffL) {
+    if (set_tile_x<T>(B, i) || set_tile_y(B, i)) {
+      add_fused<T>(B, H, l, i, P.fused);
+    } else if (nu >= 2 && d.cells() >= 100000 && d.pxy * (long)sizeof(T) <= 0x7fffffffL) {
       P.sweep.push_back(i);
       lv.push_back(&d);
       cells += d.cells();
@@ -547,14 +567,7 @@ static SmoothPlan<T> smooth_plan(pepsmg_batch* B, std::vector<Hier<T>*>& H, int 
     P.shape = Ops<T>::tall_block(cells) ? 2 : Ops<T>::large_block(cells) ? 1 : 0;
     return P;
   }
-  for (int i : rest) {
-    int tx = B->items[i].tile_x ? B->items[i].tile_x : B->opt.tile_x;
-    int ty = B->items[i].tile_y ? B->items[i].tile_y : B->opt.tile_y;
-    const bool big = H[i]->lv[l].ny >= 256;
-    if (!tx) tx = big ? Ops<T>::FTX : 64;
-    if (!ty) ty = big ? 32 : 8;
-    P.fused[sizeof(T) == 4 && tx != 64][ty == 32 ? 2 : ty == 16 ? 1 : 0].push_back(i);
-  }
+  for (int i : rest) add_fused<T>(B, H, l, i, P.fused);
   return P;
 }
 
@@ -594,7 +607,7 @@ static void rec_smooth(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, int 
       } else rec_sweep<T, 2, SW_X>(B, S, H, P.sweep, l, omega);
     }
     std::vector<int> g[2][3];
-    g[0][0] = P.sweep;
+    for (int i : P.sweep) add_fused<T>(B, H, l, i, g);
     if (it < nu) fused(g, false);
   }
   if (!P.block.empty()) {

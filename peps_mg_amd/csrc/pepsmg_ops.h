@@ -236,6 +236,10 @@ struct Ops {
   // them and b stored into d.b, 4 as 0 with x also stored into the caller's sol.
   // prefetch: planes of look-ahead of the global loads.
   int prefetch = 1;
+  // A tile or a look-ahead that is set asks for the kernel that has them:
+  // every level then runs one iteration a launch (k_rb_fused).  (FP64 tiles
+  // are 64 wide whatever tile_x says.)
+  bool single() const { return tile_y > 0 || prefetch == 2 || (sizeof(T) == 4 && tile_x > 0); }
   // the caller's padded (0:nx+1, 0:ny+1, 0:nz+1) arrays on level d, for modes 3 and 4
   void set_caller(const DevLevel<T>& d, T* sol, const T* rhs) {
     caller_lvl = d.L();
@@ -354,8 +358,8 @@ struct Ops {
   // against 42.8; mixed 128^3 (0.11) 1.55 against 1.57, 160^3 1.97 against 2.21, 256^3 3.22 against 3.78, 384^3 6.49
   // against 9.89, 512^3 13.1 against 17.5.  (A plane's row offsets are
   // 32-bit bytes.)
-  static bool sweeps(const DevLevel<T>& d) {
-    if (d.cells() < 4000000L || d.pxy * (long)sizeof(T) > 0x7fffffffL) return false;
+  bool sweeps(const DevLevel<T>& d) const {
+    if (single() || d.cells() < 4000000L || d.pxy * (long)sizeof(T) > 0x7fffffffL) return false;
     double share = 0.0;
     sweep_grid<SweepShape<T, SW_WAVES, 2, SW_X>>(d, &share);
     return share >= 0.15;
@@ -413,7 +417,7 @@ struct Ops {
   // against 0.70 ms, 64^3 0.80 against 0.99, 96^3 1.05 against 1.31, 128^3
   // 1.47 against 1.54.
   static bool blocks(long cells) { return cells <= (sizeof(T) == 8 ? 1200000L : 3000000L); }
-  static bool blocks(const DevLevel<T>& d) { return blocks(d.cells()); }
+  bool blocks(const DevLevel<T>& d) const { return !single() && blocks(d.cells()); }
   // 32 x 8 x 8 blocks of 1024 threads from 150000 cells on: less ring per cell
   // (96^3 FP64 2.14 against 2.38 ms); below, 16 x 8 x 4 keeps more CUs busy
   // (64^3 FP64 1.56 against 1.69 ms when its fine level, too, takes them)
