@@ -56,8 +56,12 @@ def _store(db):
         pass
 
 
+# part of every key: raised when kernels change what a saved measurement says
+CACHE_VERSION = 3
+
+
 def _key(kind, sdm, precision, extra=""):
-    return f"{kind}:{sdm.nx}x{sdm.ny}x{sdm.nz}:p{precision}{extra}"
+    return f"{kind}:{sdm.nx}x{sdm.ny}x{sdm.nz}:p{precision}{extra}:v{CACHE_VERSION}"
 
 
 def tune_tiles(sdm, nlevel, precision, reps=10, use_cache=True):
@@ -103,7 +107,7 @@ def tune_solver(sdm, nlevel, d_sol, d_rhs, maxiteration=2, tolerance=1e-10, omeg
     import torch
     from .multigrid import Multigrid
     db = _load() if use_cache else {}
-    key = _key("solve", sdm, precision, f":nl{nlevel}:nu{maxiteration}:v2")
+    key = _key("solve", sdm, precision, f":nl{nlevel}:nu{maxiteration}")
     if key in db:
         return db[key]
     tiles = _opts(tune_tiles(sdm, nlevel, precision, use_cache=use_cache))
