@@ -289,6 +289,11 @@ def vcycle_roofline(n, levels, t, cycles):
                      "iteration on coarse levels, so it moves fewer bytes than counted"}
 
 
+def iterations_per_launch(kernel):
+    """Red/black iterations of one launch of the smoother kernel named."""
+    return 2 if kernel.startswith("k_sweep<") or (kernel.startswith("k_block<") and ">, 2, " in kernel) else 1
+
+
 def kernel_timing(mg, enable):
     """The library's measurement hook: HIP events on the solve stream around
     every plain fused smoother launch on the finest level of the solves that
@@ -301,7 +306,9 @@ def kernel_timing(mg, enable):
     _lib.check(L.pepsmg_kernel_timing(mg.h, 0))
     tot, cnt, name = C.c_double(0), C.c_int32(0), C.c_char_p()
     _lib.check(L.pepsmg_kernel_timing_read(mg.h, C.byref(tot), C.byref(cnt), C.byref(name)))
-    return (tot.value / cnt.value if cnt.value else None), cnt.value, name.value.decode()
+    name = name.value.decode()
+    n = cnt.value // iterations_per_launch(name)   # (the library counts iterations)
+    return (tot.value / n if n else None), n, name
 
 
 def timed_solves(mg, d_x, d_b, steps, warmup, label, torch, nu=2, omega=1.0, time_smoother=False):
@@ -775,6 +782,8 @@ def main():
     avg64, n64, kin64 = r64s.smoother
     avg32, n32, kin32 = rmxs.smoother
     assert kin64 == kname64 and kin32 == kname32, (kin64, kname64, kin32, kname32)
+    # (a small level's solves may have no launch that only smooths: 0 launches, the back-to-back time)
+    avg64, avg32 = avg64 or bb64, avg32 or bb32
     achieved = nbytes64 / (avg64 * 1e-3) / 1e9
     achieved32 = nbytes32 / (avg32 * 1e-3) / 1e9
     # the bandwidth a kernel with the smoother's streams (x, b in; x out) and no
@@ -850,7 +859,7 @@ def main():
             "traffic_write": round(tr["WRITE_SIZE"]) if tr else None,
             "kernel": kname64, "kernel_down": kname64.replace("k_rb_fused<", "k_rb_fused_down<"),
             "avg_ms": avg64, "launches": n64, "bytes_per_launch": nbytes64,
-            "iterations_per_launch": 2 if kname64.startswith("k_sweep") else 1,
+            "iterations_per_launch": iterations_per_launch(kname64),
             "timing": f"HIP events on the solve stream around every plain launch on the {n}^3 level inside "
                       f"{ev_steps} FP64 solves run after the timed ones (k_sweep: two iterations a launch; "
                       "k_rb_fused: one, downward where it follows an upward one); bytes_per_launch is one "
@@ -858,11 +867,11 @@ def main():
             "stream_ceiling_gbs": round(stream_gbs, 1), "frac_of_stream_ceiling": round(achieved / stream_gbs, 4),
             "back_to_back": {"avg_ms": bb64, "frac": frac(nbytes64, bb64),
                              "note": f"{a.smoother_reps} launches in a row after {a.smoother_reps} untimed ones "
-                                     "(pepsmg_bench_smoother, alternating upward and downward), events around the whole run"}}
+                                     "(pepsmg_bench_smoother), events around the whole run"}}
     roof32 = {"achieved": round(achieved32, 1), "frac": round(achieved32 / HBM_PEAK_GBS, 4), "kernel": kname32,
               "kernel_down": kname32.replace("k_rb_fused<", "k_rb_fused_down<"),
               "avg_ms": avg32, "launches": n32, "bytes_per_launch": nbytes32,
-              "iterations_per_launch": 2 if kname32.startswith("k_sweep") else 1,
+              "iterations_per_launch": iterations_per_launch(kname32),
               "timing": f"HIP events around every launch on the {n}^3 level inside {ev_steps} mixed solves "
                         "(default options) run after the timed ones",
               "back_to_back": {"avg_ms": bb32, "frac": frac(nbytes32, bb32)}}

@@ -206,8 +206,9 @@ int pepsmg_vv_dot_device_noalloc(int32_t nx, int32_t ny, int32_t nz, const doubl
  * per-thread buffer, valid until the calling thread's next call).  As in a
  * solve, a launch that follows an upward one marches down (the symbol's
  * k_rb_fused_down twin), so the launches alternate between the two; on
- * levels where the solver runs two iterations in a launch (k_sweep), so does
- * this hook, and the time and bytes are those of such a launch. */
+ * levels where the solver takes two iterations in a launch (k_sweep on large
+ * ones, k_block on small ones), so does this hook, and the time and bytes are
+ * those of such a launch. */
 int pepsmg_bench_smoother(pepsmg_ctx *ctx, int32_t precision, int32_t reps, double omega,
                           double *avg_ms, double *bytes, const char **kernel_name);
 
@@ -216,13 +217,14 @@ int pepsmg_bench_smoother(pepsmg_ctx *ctx, int32_t precision, int32_t reps, doub
  * finest level (FP64; in precision 1 the FP32 smoother) with HIP events on
  * the solve stream, and clears the totals; 0 stops.  Up to 256 launches per
  * solve are timed, both upward and downward ones (k_rb_fused_down); where
- * the finest level's plain launches are two iterations each (k_sweep), those;
- * on levels smoothed by blocks (k_block) every launch, counted with its
- * iterations. */
+ * the solve takes two iterations in a launch (k_sweep, k_block), the launches
+ * of two that start from x and do nothing else beside them.  A small level
+ * may have none: its launches also prolongate, restrict or form the norm. */
 int pepsmg_kernel_timing(pepsmg_ctx *ctx, int32_t enable);
 
 /* Totals since the last pepsmg_kernel_timing(ctx, 1) (kept when timing is
- * switched off): summed duration of the timed launches (ms), their number,
+ * switched off): summed duration of the timed launches (ms), the iterations
+ * they ran (two each for k_sweep and k_block symbols that say so, else one),
  * and the kernel's symbol (valid until timing is next switched on). */
 int pepsmg_kernel_timing_read(const pepsmg_ctx *ctx, double *total_ms, int32_t *launches,
                               const char **kernel_name);

@@ -151,7 +151,7 @@ struct KernelTimer {
   bool on = false;
   const void* level = nullptr;   // the DevLevel whose plain fused launches are timed
   std::vector<hipEvent_t> ev;    // pairs (before, after)
-  std::vector<int> count;        // what a pair's launch counts for (k_block: its iterations)
+  std::vector<int> count;        // iterations of a pair's launch
   int used = 0;                  // events recorded in the solve in progress
   double total_ms = 0.0;
   long launches = 0;

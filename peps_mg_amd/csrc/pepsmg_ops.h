@@ -251,8 +251,10 @@ struct Ops {
     caller_b = rhs + o;
   }
 
-  // measurement hook: plain launches on the timer's level are bracketed by events
+  // measurement hook: plain launches on the timer's level are bracketed by
+  // events: those of the one kernel smoother_name names, nothing else
   KernelTimer* timer = nullptr;
+  int timed_nit = 1;             // iterations of such a launch
   void timer_begin(const DevLevel<T>& d, int mode, bool& timed) {
     timed = timer && timer->wants(&d, mode);
     if (timed) hipEventRecord(timer->ev[timer->used], s);
@@ -276,7 +278,7 @@ struct Ops {
     int ty = ty_used(d);
     const bool down = next_down(d, mode);
     bool timed;
-    timer_begin(d, timer && (blocks(d) || sweeps(d)) ? 1 : mode, timed);   // (where k_sweep is the plain kernel, it alone is timed)
+    timer_begin(d, timed_nit == 1 && !(timer && blocks(d)) ? mode : 1, timed);
     if (sizeof(T) == 4 && tx_used(d) == 64) fused_tx<64>(d, omega, mode, ty, partial, down);
     else fused_tx<FTX>(d, omega, mode, ty, partial, down);
     timer_end(timed);
@@ -288,7 +290,7 @@ struct Ops {
     int ty = ty_used(d);
     const bool down = next_down(d, 0);
     bool timed;
-    timer_begin(d, timer && (blocks(d) || sweeps(d)) ? 1 : 0, timed);
+    timer_begin(d, timed_nit == 1 && !(timer && blocks(d)) ? 0 : 1, timed);
     if (sizeof(T) == 4 && tx_used(d) == 64) fused_tx<64>(d, omega, 0, ty, nullptr, down);
     else fused_tx<FTX>(d, omega, 0, ty, nullptr, down);
     timer_end(timed);
@@ -401,10 +403,10 @@ struct Ops {
     A.G = sweep_grid<S>(d);
     const unsigned nb = (unsigned)((A.G.gx * A.G.gy * A.G.nch + 7) / 8 * 8);
     bool timed;
-    timer_begin(d, PRE == SW_X && !to_caller ? 0 : 1, timed);
+    timer_begin(d, PRE == SW_X && !to_caller && timed_nit == NIT ? 0 : 1, timed);
     set_dynamic_lds((const void*)k_sweep<T, SW_WAVES, NIT, PRE>, S::LDS * sizeof(T));   // a failure surfaces at the solve's end
     hipLaunchKernelGGL((k_sweep<T, SW_WAVES, NIT, PRE>), dim3(nb), dim3(S::THREADS), S::LDS * sizeof(T), s, A);
-    timer_end(timed);
+    timer_end(timed, NIT);
     d.fused_up = true;
     std::swap(d.x, d.x2);
   }
@@ -478,7 +480,7 @@ struct Ops {
     A.partial = partial;
     const int nb = block_count<B>(d);
     bool timed;
-    timer_begin(d, 0, timed);
+    timer_begin(d, PRE == SW_X && !NORM && !REST && timed_nit == NIT ? 0 : 1, timed);
     if (S::LDS * sizeof(T) > 65536)
       set_dynamic_lds((const void*)k_block<T, B, NIT, PRE, NORM, REST>, S::LDS * sizeof(T));
     hipLaunchKernelGGL((k_block<T, B, NIT, PRE, NORM, REST>), dim3((unsigned)nb), dim3(B::NT), S::LDS * sizeof(T), s, A);
@@ -582,14 +584,25 @@ struct Ops {
     for (; it < nu; it++) fused_iter(d, omega, (it == 0 && zero_start) ? 1 : (it == nu - 1 && last_mode ? last_mode : 0));
   }
 
-  // symbol of the plain smoother kernel iterate launches on level d
-  void smoother_name(const DevLevel<T>& d, char* buf, size_t n) const {
+  // iterations of a plain launch of nu iterations on level d
+  int launch_nit(const DevLevel<T>& d, int nu) const { return nu >= 2 && (blocks(d) || sweeps(d)) ? 2 : 1; }
+  // symbol of the plain smoother kernel iterate launches on level d for nu iterations
+  void smoother_name(const DevLevel<T>& d, int nu, char* buf, size_t n) const {
+    const char* t = sizeof(T) == 8 ? "double" : "float";
+    const int nit = launch_nit(d, nu);
     if (blocks(d)) {
-      std::snprintf(buf, n, "k_block<%s", sizeof(T) == 8 ? "double" : "float");
+      auto name = [&](auto b) {
+        using B = decltype(b);
+        std::snprintf(buf, n, "k_block<%s, pepsmg::BlockTile<%d, %d, %d, %d>, %d, %d, false, false>", t, B::BX, B::BY,
+                      B::BZ, B::NT, nit, (int)SW_X);
+      };
+      if (tall_block(d.cells())) name(BlockTall());
+      else if (large_block(d.cells())) name(BlockLarge());
+      else name(BlockSmall());
       return;
     }
-    if (sweeps(d)) {
-      std::snprintf(buf, n, "k_sweep<%s, %d, 2, 0>", sizeof(T) == 8 ? "double" : "float", SW_WAVES);
+    if (nit == 2) {
+      std::snprintf(buf, n, "k_sweep<%s, %d, 2, %d>", t, SW_WAVES, (int)SW_X);
       return;
     }
     const int ty = ty_used(d);

@@ -387,14 +387,16 @@ void pepsmg_ctx::release() {
 
 namespace pepsmg {
 
-// Measurement hook: time the plain fused launches on level d of this solve.
+// Measurement hook: time the plain fused launches on level d of this solve,
+// nu iterations at a time.
 template <typename T>
-static void timer_attach(pepsmg_ctx* c, Ops<T>& op, DevLevel<T>& d) {
+static void timer_attach(pepsmg_ctx* c, Ops<T>& op, DevLevel<T>& d, int nu) {
   if (!c->timer.on) return;
+  op.timed_nit = op.launch_nit(d, nu);
   op.timer = &c->timer;
   c->timer.level = &d;
   c->timer.used = 0;
-  op.smoother_name(d, c->timer.name, sizeof c->timer.name);
+  op.smoother_name(d, nu, c->timer.name, sizeof c->timer.name);
 }
 
 // Adds the bracketed launches of the finished solve to the totals.
@@ -624,7 +626,7 @@ static int solve_fp64(pepsmg_ctx* c, int nu, double tol, double omega, pepsmg_st
   op.tile_y = c->opt.tile_y;
   op.prefetch = c->opt.fused_smoother == 2 ? 2 : 1;
   op.tile_x = c->opt.tile_x;
-  timer_attach(c, op, h.lv[0]);
+  timer_attach(c, op, h.lv[0], nu);
   CgBufs<double>* cg = nullptr;
   if (c->opt.smoother == 1) {
     cg = &c->cg64;
@@ -781,7 +783,6 @@ static int solve_mixed(pepsmg_ctx* c, int nu, double tol, double omega, std::vec
   op.tile_y = c->opt.tile_y;
   op.prefetch = c->opt.fused_smoother == 2 ? 2 : 1;
   op.tile_x = c->opt.tile_x;
-  timer_attach(c, op, g.lv[0]);
   CgBufs<float>* cg = nullptr;
   if (c->opt.smoother == 1) {
     cg = &c->cg32;
@@ -862,6 +863,7 @@ static int solve_mixed(pepsmg_ctx* c, int nu, double tol, double omega, std::vec
   // maxiteration) and inner_nu_post (or the pre-smoothing count)
   const int nui = c->opt.inner_nu > 0 ? c->opt.inner_nu : nu;
   const int nup = c->opt.inner_nu_post > 0 ? c->opt.inner_nu_post : nui;
+  timer_attach(c, op, g.lv[0], std::max(nui, nup));
   // The host reads each norm while the GPU already runs the next step's
   // first pre-smoothing and restriction (which need only r32, and touch no FP64 array), so
   // the read-back leaves no gap; skipped when the step is predicted to stop.
@@ -1176,7 +1178,7 @@ int pepsmg_bench_smoother(pepsmg_ctx* c, int32_t precision, int32_t reps, double
   float ms = 0;
   double n = 0;
   const bool fused = c->opt.fused_smoother != 0;
-  // fused: a launch (two iterations where k_sweep is the solver's kernel,
+  // fused: a launch (two iterations where the solver takes two at a time,
   // else one) reads x and b and writes x once (3 n elements); colour sweep:
   // reads x and b, writes half of x (2 n)
   auto run = [&](auto& op, auto& d, const char* tname) -> int {
@@ -1186,7 +1188,7 @@ int pepsmg_bench_smoother(pepsmg_ctx* c, int32_t precision, int32_t reps, double
     using T = typename std::remove_reference<decltype(d.x[0])>::type;
     auto body = [&]() {
       for (int q = 0; q < reps; q++) {
-        if (fused && op.blocks(d)) op.template block<1, SW_X>(d, nullptr, (T)omega);
+        if (fused && op.blocks(d)) op.template block<2, SW_X>(d, nullptr, (T)omega);
         else if (fused && op.sweeps(d)) op.template sweep<2, SW_X>(d, nullptr, (T)omega);
         else if (fused) op.fused_iter(d, (T)omega, 0);
         else op.smooth_colour(d, d.b, d.x, (T)omega, q & 1, false);
@@ -1198,7 +1200,7 @@ int pepsmg_bench_smoother(pepsmg_ctx* c, int32_t precision, int32_t reps, double
     HIP_TRY(hipEventRecord(c->ev1, c->stream));
     n = (double)d.cells();
     if (fused)
-      op.smoother_name(d, name, sizeof name);
+      op.smoother_name(d, 2, name, sizeof name);
     else
       std::snprintf(name, sizeof name, "k_rb_colour<%s, false>", tname);
     return PEPSMG_OK;
