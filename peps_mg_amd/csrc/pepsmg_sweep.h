@@ -188,8 +188,9 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
   }
   // Planes zlo .. zhi share their z coefficients: there the divisors are
   // kept.  FP64: c0 and 1 / c0; FP32: omega / c0 alone.  Cells outside the
-  // level get the factor 0, which leaves them 0 (in FP32 also beside an
-  // infinity or a NaN: the product with 0 is taken as 0).
+  // level get the factor 0, which leaves them 0; FP32 also selects by lev
+  // (beside an infinity or a NaN the product with 0 is a NaN).
+  bool lev[R][2];
   T dv[F64 ? R : 1][2], rv[R][2];
   bool kept = A.zhi >= A.zlo;
 #pragma unroll
@@ -197,6 +198,7 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
 #pragma unroll
     for (int c = 0; c < 2; c++) {
       const bool in = (c ? in1 : in0) && j0 + r <= L.ny;
+      lev[r][c] = in;
       const T c0 = -(c1[c] + c2[c] + c3[r] + c4[r] + A.c5u + A.c6u);
       if constexpr (F64) {
         dv[r][c] = c0;
@@ -470,7 +472,10 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
           for (int r = 0; r < R; r++) put(r, q[r]);
         } else if constexpr (FAST) {
 #pragma unroll
-          for (int r = 0; r < R; r++) put(r, diff(r, A.c5u, A.c6u) * rv[r][cell(r)]);
+          for (int r = 0; r < R; r++) {
+            const T q = diff(r, A.c5u, A.c6u) * rv[r][cell(r)];
+            put(r, lev[r][cell(r)] ? q : T(0));
+          }
         } else {
           const T c5 = ldc(L.cwz, k), c6 = ldc(L.cez, k);
 #pragma unroll
