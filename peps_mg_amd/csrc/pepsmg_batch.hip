@@ -19,9 +19,10 @@
 // refinement step).  A replay is one V-cycle (FP64) or one refinement step
 // (mixed); the host reads one counter of still-active items per replay.
 // In FP64 the values an item gets are exactly those of its single-grid solve
-// with the same options.  Mixed precision: which smoother kernel serves a
-// level follows the batch's cells, not the item's, and the FP32 kernels round
-// differently; the final refinement step always runs inner_cycles cycles.
+// with the same options.  In mixed precision, too, they do not depend on what
+// else is in the batch, whose cells decide which smoother kernels run: these
+// round alike.  (There the final refinement step always runs inner_cycles
+// cycles, where the single-grid solver may run fewer.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

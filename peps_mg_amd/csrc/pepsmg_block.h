@@ -137,8 +137,10 @@ __device__ __forceinline__ void block_tile(const BlockArgs<T>& A, int bid) {
       const T* p = axis == 0 ? A.W.px_ : axis == 1 ? A.W.py_ : A.W.pz_;
       const T* m = axis == 0 ? A.W.nx_ : axis == 1 ? A.W.ny_ : A.W.nz_;
       const int g = min(max(f, 1), n);
-      pw[2 * t] = g & 1 ? p[g] : m[g];
-      pw[2 * t + 1] = g & 1 ? p[g + 1] : m[g - 1];
+      T ws = g & 1 ? p[g] : m[g], wn = g & 1 ? p[g + 1] : m[g - 1];
+      if constexpr (!F64) interp_norm(ws, wn);
+      pw[2 * t] = ws;
+      pw[2 * t + 1] = wn;
     }
   }
   // REST: the thread's coarse cell and its weights
@@ -185,10 +187,16 @@ __device__ __forceinline__ void block_tile(const BlockArgs<T>& A, int bid) {
       for (int c = 0; c < 2; c++) {
         const T sx = wx[2 * c], nx = wx[2 * c + 1];
         const int dx = c ? 1 : -1;
-        const T num = sx * sy * sz * P[0] + nx * sy * sz * P[dx] + sx * ny * sz * P[dy] + sx * sy * nz * P[dz] +
-                      nx * ny * sz * P[dx + dy] + nx * sy * nz * P[dx + dz] + sx * ny * nz * P[dy + dz] +
-                      nx * ny * nz * P[dx + dy + dz];
-        const T add = num / ((sx + nx) * (sy + ny) * (sz + nz));
+        T add;
+        if constexpr (F64) {
+          const T num = sx * sy * sz * P[0] + nx * sy * sz * P[dx] + sx * ny * sz * P[dy] + sx * sy * nz * P[dz] +
+                        nx * ny * sz * P[dx + dy] + nx * sy * nz * P[dx + dz] + sx * ny * nz * P[dy + dz] +
+                        nx * ny * nz * P[dx + dy + dz];
+          add = num / ((sx + nx) * (sy + ny) * (sz + nz));
+        } else {
+          add = interp_zxy(sz, nz, sx, nx, sy, ny, P[0], P[dx], P[dy], P[dx + dy], P[dz], P[dz + dx], P[dz + dy],
+                           P[dz + dx + dy]);
+        }
         if (c) xv[p].y = xv[p].y + add;
         else xv[p].x = xv[p].x + add;
       }
@@ -203,19 +211,6 @@ __device__ __forceinline__ void block_tile(const BlockArgs<T>& A, int bid) {
   }
   __syncthreads();
 
-  // neighbours of cell c of pair p: own array at +- a row or plane, the other
-  // array at the pair and beside it
-  auto temp = [&](int p, int c, T a1, T a2, T c3, T c4, T c5, T c6) -> T {
-    const T* o = xs + c * NP + id[p];
-    const T* w = xs + (1 - c) * NP + id[p] - (1 - c);
-    if constexpr (F64) return a1 * w[0] + a2 * w[1] + c3 * o[-PX] + c4 * o[PX] + c5 * o[-PX * RY] + c6 * o[PX * RY];
-    T d = a1 * w[0];
-    d = sw_fma(a2, w[1], d);
-    d = sw_fma(c3, o[-PX], d);
-    d = sw_fma(c4, o[PX], d);
-    d = sw_fma(c5, o[-PX * RY], d);
-    return sw_fma(c6, o[PX * RY], d);
-  };
   if constexpr (NORM) {
     double acc = 0.0;
 #pragma unroll
@@ -251,13 +246,16 @@ __device__ __forceinline__ void block_tile(const BlockArgs<T>& A, int bid) {
       const T* kx = cx + 2 * (2 * (at[p] & 255) + c);
       const T a1 = kx[0], a2 = kx[1], bb = c ? bv[p].y : bv[p].x;
       T* o = xs + (c ? NP : 0) + id[p];
-      const T tm = PRE == SW_ZERO && s == 1 ? T(0) : temp(p, c, a1, a2, c3, c4, c5, c6);
-      const T xold = PRE == SW_ZERO && s == 1 ? T(0) : o[0];
-      if constexpr (F64) {
-        o[0] = sor_update(A.omega, bb, tm, diag(a1, a2, c3, c4, c5, c6), xold);
+      // neighbours: own array at +- a row or plane, the other array at the pair and beside it
+      const T* w = xs + (c ? 0 : NP) + id[p] - (c ? 0 : 1);
+      if (PRE == SW_ZERO && s == 1) {
+        o[0] = sor_zero(A.omega, bb, diag(a1, a2, c3, c4, c5, c6));
+      } else if constexpr (F64) {
+        const T tm = a1 * w[0] + a2 * w[1] + c3 * o[-PX] + c4 * o[PX] + c5 * o[-PX * RY] + c6 * o[PX * RY];
+        o[0] = sor_update(A.omega, bb, tm, diag(a1, a2, c3, c4, c5, c6), o[0]);
       } else {
-        const T f = A.omega * __builtin_amdgcn_rcpf(a1 + a2 + (c3 + c4) + (c5 + c6));
-        o[0] = sw_fma(tm - bb, f, (T(1) - A.omega) * xold);
+        const T tm = sor_temp(SorC<T>{a1, a2, c3, c4, c5, c6}, w[0], w[1], o[-PX], o[PX], o[-PX * RY], o[PX * RY]);
+        o[0] = sor_next(A.omega, bb, tm, sor_factor(A.omega, diag(a1, a2, c3, c4, c5, c6)), o[0]);
       }
     }
     if (s < 2 * NIT) __syncthreads();

@@ -62,6 +62,11 @@ __device__ __forceinline__ void prolong_march_block(int bid, T* __restrict__ xf,
     wny[q] = act[q] ? (jodd ? W.py_[gj + 1] : W.ny_[gj - 1]) : T(0);
     cjr[q] = jc - jc0 + 1;
     njr[q] = (jodd ? jc - 1 : jc + 1) - jc0 + 1;
+    if constexpr (sizeof(T) == 4) {
+      interp_norm(wsa[q], wna[q]);
+      interp_norm(wsb[q], wnb[q]);
+      interp_norm(wsy[q], wny[q]);
+    }
   }
 
   // Coarse and fine planes load from clamped in-bounds addresses with no
@@ -130,6 +135,7 @@ __device__ __forceinline__ void prolong_march_block(int bid, T* __restrict__ xf,
       issue_f(xpre[h], f + 2);
       T wsz = (h == 0) ? ldc(W.pz_, f) : ldc(W.nz_, f);
       T wnz = (h == 0) ? ldc(W.pz_, f + 1) : ldc(W.nz_, f - 1);
+      if constexpr (sizeof(T) == 4) interp_norm(wsz, wnz);
       T(*P)[CX] = sc[kc & 3];
       T(*N)[CX] = sc[(h == 0 ? kc - 1 : kc + 1) & 3];
 #pragma unroll
@@ -141,18 +147,28 @@ __device__ __forceinline__ void prolong_march_block(int bid, T* __restrict__ xf,
         {
           T sx = wsa[q], nx = wna[q];
           int ci = lcx, ni = lcx - 1;
-          T num = sx * sy * wsz * P[cj][ci] + nx * sy * wsz * P[cj][ni] + sx * ny * wsz * P[nj][ci] +
-                  sx * sy * wnz * N[cj][ci] + nx * ny * wsz * P[nj][ni] + nx * sy * wnz * N[cj][ni] +
-                  sx * ny * wnz * N[nj][ci] + nx * ny * wnz * N[nj][ni];
-          xv[q].x = xv[q].x + num / ((sx + nx) * (sy + ny) * (wsz + wnz));
+          if constexpr (sizeof(T) == 4) {
+            xv[q].x = xv[q].x + interp_zxy(wsz, wnz, sx, nx, sy, ny, P[cj][ci], P[cj][ni], P[nj][ci], P[nj][ni],
+                                           N[cj][ci], N[cj][ni], N[nj][ci], N[nj][ni]);
+          } else {
+            T num = sx * sy * wsz * P[cj][ci] + nx * sy * wsz * P[cj][ni] + sx * ny * wsz * P[nj][ci] +
+                    sx * sy * wnz * N[cj][ci] + nx * ny * wsz * P[nj][ni] + nx * sy * wnz * N[cj][ni] +
+                    sx * ny * wnz * N[nj][ci] + nx * ny * wnz * N[nj][ni];
+            xv[q].x = xv[q].x + num / ((sx + nx) * (sy + ny) * (wsz + wnz));
+          }
         }
         if (two[q]) {   // second cell (even i): parent lcx, neighbour lcx+1
           T sx = wsb[q], nx = wnb[q];
           int ci = lcx, ni = lcx + 1;
-          T num = sx * sy * wsz * P[cj][ci] + nx * sy * wsz * P[cj][ni] + sx * ny * wsz * P[nj][ci] +
-                  sx * sy * wnz * N[cj][ci] + nx * ny * wsz * P[nj][ni] + nx * sy * wnz * N[cj][ni] +
-                  sx * ny * wnz * N[nj][ci] + nx * ny * wnz * N[nj][ni];
-          xv[q].y = xv[q].y + num / ((sx + nx) * (sy + ny) * (wsz + wnz));
+          if constexpr (sizeof(T) == 4) {
+            xv[q].y = xv[q].y + interp_zxy(wsz, wnz, sx, nx, sy, ny, P[cj][ci], P[cj][ni], P[nj][ci], P[nj][ni],
+                                           N[cj][ci], N[cj][ni], N[nj][ci], N[nj][ni]);
+          } else {
+            T num = sx * sy * wsz * P[cj][ci] + nx * sy * wsz * P[cj][ni] + sx * ny * wsz * P[nj][ci] +
+                    sx * sy * wnz * N[cj][ci] + nx * ny * wsz * P[nj][ni] + nx * sy * wnz * N[cj][ni] +
+                    sx * ny * wnz * N[nj][ci] + nx * ny * wnz * N[nj][ni];
+            xv[q].y = xv[q].y + num / ((sx + nx) * (sy + ny) * (wsz + wnz));
+          }
         }
         long q0 = lidx(F, ia, j0 + ly[q], f);
         if (two[q]) st_stream_pair(xf + q0, xv[q].x, xv[q].y);

@@ -102,15 +102,40 @@ struct FusedGrid {
   int order = 0;   // workgroup order (fused_xcd_bid)
 };
 
-// omega * (b - temp) / c0 + (1 - omega) * xold, the reference's SOR update
-// (src/rbgs_poisson_matrix.f90:250).  FP64 divides exactly (bit-identical
-// results); the FP32 inner solver of the mixed-precision path multiplies by
-// the hardware reciprocal (1 ulp), which leaves its convergence unchanged.
+// The reference's SOR update (src/rbgs_poisson_matrix.f90:244-250): in FP64
+// its expression, operand order and division (bit-identical results),
+//   omega (b - (c1 xw + c2 xe + c3 xs + c4 xn + c5 xb + c6 xt)) / c0 + (1 - omega) xold.
+// The FP32 inner solver of the mixed-precision path fuses each product into
+// the difference and multiplies by omega and the hardware reciprocal of c0 (1
+// ulp), which leaves its convergence unchanged.  Every FP32 smoother kernel
+// (k_rb_fused, k_block, k_sweep) forms these values by these steps, so they
+// do not depend on which of them serves a level.
+template <typename T>
+struct SorC {                                        // c1 .. c6
+  T w, e, s, n, b, t;
+};
 __device__ __forceinline__ double sor_update(double omega, double bv, double temp, double c0, double xold) {
   return omega * (bv - temp) / c0 + (1.0 - omega) * xold;
 }
-__device__ __forceinline__ float sor_update(float omega, float bv, float temp, float c0, float xold) {
-  return omega * (bv - temp) * __builtin_amdgcn_rcpf(c0) + (1.0f - omega) * xold;
+// c1 xw + ... + c6 xt
+__device__ __forceinline__ float sor_temp(const SorC<float>& c, float xw, float xe, float xs, float xn, float xb,
+                                          float xt) {
+  float d = c.w * xw;
+  d = __builtin_fmaf(c.e, xe, d);
+  d = __builtin_fmaf(c.s, xs, d);
+  d = __builtin_fmaf(c.n, xn, d);
+  d = __builtin_fmaf(c.b, xb, d);
+  return __builtin_fmaf(c.t, xt, d);
+}
+__device__ __forceinline__ float sor_factor(float omega, float c0) { return omega * __builtin_amdgcn_rcpf(c0); }
+__device__ __forceinline__ float sor_next(float omega, float bv, float temp, float f, float xold) {
+  return __builtin_fmaf(1.0f - omega, xold, (bv - temp) * f);
+}
+// the update from x = 0 (the products sum to +0)
+template <typename T>
+__device__ __forceinline__ T sor_zero(T omega, T bv, T c0) {
+  if constexpr (sizeof(T) == 8) return sor_update(omega, bv, T(0), c0, T(0));
+  else return bv * sor_factor(omega, c0);
 }
 
 // Modes 0 and 4 on tiles of 2048 cells or more (one or two blocks per CU
@@ -148,6 +173,7 @@ __device__ __forceinline__ double rb_fused_body(T* __restrict__ xo, const T* __r
                                                 const T* __restrict__ b, const Lvl<T>& L, T omega, int i0, int j0,
                                                 int k0, int k1, T* __restrict__ sx, T* __restrict__ sr,
                                                 T* __restrict__ sbk, const Lvl<T>& U, T* __restrict__ ext) {
+  constexpr bool F64 = sizeof(T) == 8;
   constexpr bool NORM = MODE == 2 || MODE == 3;   // partial sums of (b - A x_in)^2
   constexpr bool CALLER_IN = MODE == 3;           // x_in and b in the caller's layout U
   constexpr bool CALLER_OUT = MODE == 4;          // x_out also into the caller's layout U
@@ -344,15 +370,20 @@ __device__ __forceinline__ double rb_fused_body(T* __restrict__ xo, const T* __r
         T c1 = r_c1[q][Z], c2 = r_c2[q][Z], c3 = r_c3[q], c4 = r_c4[q];
         T c0 = -(r_s4[q][Z] + c5 + c6);
         if (ZB) {   // black neighbours and the old value are 0 (their products sum to +0)
-          v = sor_update(omega, X0[ss], T(0), c0, T(0));
+          v = sor_zero(omega, X0[ss], c0);
         } else {
-          T temp = c1 * X0[oo] + c2 * X0[oo + 1] + c3 * X0[ss - RP] + c4 * X0[ss + RP] + c5 * Xm[ss] + c6 * Xp[ss];
+          T temp;
+          if constexpr (F64)
+            temp = c1 * X0[oo] + c2 * X0[oo + 1] + c3 * X0[ss - RP] + c4 * X0[ss + RP] + c5 * Xm[ss] + c6 * Xp[ss];
+          else
+            temp = sor_temp(SorC<T>{c1, c2, c3, c4, c5, c6}, X0[oo], X0[oo + 1], X0[ss - RP], X0[ss + RP], Xm[ss], Xp[ss]);
           T bred = bv[q];
           if (PB) {
             const T p0 = brp[slot][q].x, p1 = brp[slot][q].y;
             bred = r_first[q][Z] ? p0 : p1;
           }
-          v = sor_update(omega, bred, temp, c0, X0[ss]);
+          if constexpr (F64) v = sor_update(omega, bred, temp, c0, X0[ss]);
+          else v = sor_next(omega, bred, temp, sor_factor(omega, c0), X0[ss]);
         }
       }
       if (t + q * NT < QP) r[r_q[q]] = v;
@@ -382,9 +413,19 @@ __device__ __forceinline__ double rb_fused_body(T* __restrict__ xo, const T* __r
         const int ow = b_ow[q][Z];
         T c1 = b_c1[q][Z], c2 = b_c2[q][Z], c3 = b_c3[q], c4 = b_c4[q];
         T c0 = -(b_s4[q][Z] + c5 + c6);
-        T temp = c1 * r0[ow] + c2 * r0[ow + 1] + c3 * r0[row - RP] + c4 * r0[row + RP] + c5 * rm[row] + c6 * rp[row];
-        if (ZB) vb = sor_update(omega, X0[b_xc[q][Z]], temp, c0, T(0));   // X0: b of plane k
-        else vb = sor_update(omega, PB ? sb[min(t + q * NT, TY * TP - 1)] : bv[q], temp, c0, X0[b_xc[q][Z]]);
+        T temp;
+        if constexpr (F64)
+          temp = c1 * r0[ow] + c2 * r0[ow + 1] + c3 * r0[row - RP] + c4 * r0[row + RP] + c5 * rm[row] + c6 * rp[row];
+        else
+          temp = sor_temp(SorC<T>{c1, c2, c3, c4, c5, c6}, r0[ow], r0[ow + 1], r0[row - RP], r0[row + RP], rm[row], rp[row]);
+        if constexpr (F64) {
+          if (ZB) vb = sor_update(omega, X0[b_xc[q][Z]], temp, c0, T(0));   // X0: b of plane k
+          else vb = sor_update(omega, PB ? sb[min(t + q * NT, TY * TP - 1)] : bv[q], temp, c0, X0[b_xc[q][Z]]);
+        } else {
+          const T f = sor_factor(omega, c0);
+          if (ZB) vb = (X0[b_xc[q][Z]] - temp) * f;
+          else vb = sor_next(omega, PB ? sb[min(t + q * NT, TY * TP - 1)] : bv[q], temp, f, X0[b_xc[q][Z]]);
+        }
       }
       T vr = r0[row];
       const bool bf = Z ? !b_odd[q] : b_odd[q];   // black is the first cell iff gj + k odd

@@ -245,6 +245,26 @@ __global__ void k_restrict(T* __restrict__ bc, const T* __restrict__ xf, const T
 // The eight terms are summed in the reference order (self/neighbour per axis:
 // sss, nss, sns, ssn, nns, nsn, snn, nnn) and divided by the product of the
 // per-axis weight sums.
+//
+// On levels that halve every axis the FP32 kernels (k_prolong_march, k_block,
+// k_sweep) divide each axis's weights by their sum (interp_norm) and
+// interpolate along z, then x, then y: fewer operations, and the same values
+// whichever of them serves a level.
+__device__ __forceinline__ void interp_norm(float& ws, float& wn) {
+  const float t = ws + wn;
+  ws = ws / t;
+  wn = wn / t;
+}
+// weights f (parent) and g (neighbour) of each axis; coarse values p<y><x> on
+// the parent's plane and n<y><x> on the neighbour's (0: parent, 1: neighbour)
+__device__ __forceinline__ float interp_zxy(float fz, float gz, float fx, float gx, float fy, float gy, float p00,
+                                            float p01, float p10, float p11, float n00, float n01, float n10,
+                                            float n11) {
+  auto lerp = [](float f, float a, float g, float b) { return __builtin_fmaf(g, b, f * a); };
+  const float h0 = lerp(fx, lerp(fz, p00, gz, n00), gx, lerp(fz, p01, gz, n01));
+  const float h1 = lerp(fx, lerp(fz, p10, gz, n10), gx, lerp(fz, p11, gz, n11));
+  return lerp(fy, h0, gy, h1);
+}
 template <typename T>
 __device__ __forceinline__ void prolong_axis(const T* p, const T* n, int s, int f, int& c, int& nb, T& ws,
                                              T& wn) {

@@ -205,7 +205,7 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
         rv[r][c] = in ? 1.0 / c0 : 0.0;
         kept = kept && (!in || kd_divisor(c0));
       } else {
-        rv[r][c] = in ? A.omega / c0 : T(0);
+        rv[r][c] = in ? sor_factor(A.omega, c0) : T(0);
       }
     }
   }
@@ -430,7 +430,7 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
           for (int r = 0; r < R; r++) bv[r] = src[r * NT];
         }
         // b - (c1 xw + c2 xe + c3 xs + c4 xn + c5 xb + c6 xt): the reference's
-        // order in FP64; FP32 fuses each product into the difference
+        // order in FP64; FP32 as sor_temp
         auto diff = [&](int r, T c5, T c6) -> T {
           const int c = cell(r);
           if (Z) return bv[r] - T(0);
@@ -442,12 +442,7 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
           if constexpr (F64) {
             return bv[r] - (c1[c] * xw + c2[c] * xe + c3[r] * xs + c4[r] * xn + c5 * xb + c6 * xt);
           } else {
-            T d = sw_fma(-c1[c], xw, bv[r]);
-            d = sw_fma(-c2[c], xe, d);
-            d = sw_fma(-c3[r], xs, d);
-            d = sw_fma(-c4[r], xn, d);
-            d = sw_fma(-c5, xb, d);
-            return sw_fma(-c6, xt, d);
+            return bv[r] - sor_temp(SorC<T>{c1[c], c2[c], c3[r], c4[r], c5, c6}, xw, xe, xs, xn, xb, xt);
           }
         };
         auto put = [&](int r, T q) {                 // q: omega (b - ...) / c0
@@ -484,7 +479,7 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
             const T c0 = -(sw_fresh_v(c1[c]) + c2[c] + c3[r] + c4[r] + c5 + c6);
             T q;
             if constexpr (F64) q = A.omega * diff(r, c5, c6) / c0;
-            else q = A.omega * diff(r, c5, c6) * __builtin_amdgcn_rcpf(c0);
+            else q = diff(r, c5, c6) * sor_factor(A.omega, c0);
             put(r, sw_fresh_v(rv[r][c]) != T(0) ? q : T(0));
           }
         }
