@@ -612,17 +612,21 @@ static void rec_smooth(pepsmg_batch* B, Sched& S, std::vector<Hier<T>*>& H, int 
     if (it < nu) fused(g, false);
   }
   if (!P.block.empty()) {
+    auto prolonged = [&](auto Bc, auto nit) {
+      if constexpr (Ops<T>::block_shape(decltype(Bc)(), SW_PROLONG))
+        rec_block<T, decltype(Bc), decltype(nit)::value, SW_PROLONG>(B, S, H, P.block, l, omega);
+    };
     auto block = [&](auto Bc) {
       using Bl = decltype(Bc);
       for (int it = 0; it < nu; it += 2) {
         const bool z = it == 0 && zero, p = it == 0 && pb;
         if (nu - it >= 2) {
           if (z) rec_block<T, Bl, 2, SW_ZERO>(B, S, H, P.block, l, omega);
-          else if (p) rec_block<T, Bl, 2, SW_PROLONG>(B, S, H, P.block, l, omega);
+          else if (p) prolonged(Bc, std::integral_constant<int, 2>());
           else rec_block<T, Bl, 2, SW_X>(B, S, H, P.block, l, omega);
         } else {
           if (z) rec_block<T, Bl, 1, SW_ZERO>(B, S, H, P.block, l, omega);
-          else if (p) rec_block<T, Bl, 1, SW_PROLONG>(B, S, H, P.block, l, omega);
+          else if (p) prolonged(Bc, std::integral_constant<int, 1>());
           else rec_block<T, Bl, 1, SW_X>(B, S, H, P.block, l, omega);
         }
       }

@@ -420,21 +420,31 @@ struct Ops {
   // 1.47 against 1.54.
   static bool blocks(long cells) { return cells <= (sizeof(T) == 8 ? 1200000L : 3000000L); }
   bool blocks(const DevLevel<T>& d) const { return !single() && blocks(d.cells()); }
-  // 32 x 8 x 8 blocks of 1024 threads from 150000 cells on: less ring per cell
-  // (96^3 FP64 2.14 against 2.38 ms); below, 16 x 8 x 4 keeps more CUs busy
-  // (64^3 FP64 1.56 against 1.69 ms when its fine level, too, takes them)
-  static bool large_block(long cells) { return cells > (sizeof(T) == 8 ? 300000L : 150000L); }
+  // 32 x 8 x 8 blocks of 1024 threads from 300000 cells on in FP64 and 150000
+  // in FP32: less ring per cell (96^3 FP64 2.14 against 2.38 ms); below,
+  // 16 x 8 x 4 keeps more CUs busy (64^3 FP64 1.56 against 1.69 ms when its
+  // fine level, too, takes them)
+  static constexpr long LARGE_BLOCK = sizeof(T) == 8 ? 300000 : 150000;
+  static bool large_block(long cells) { return cells > LARGE_BLOCK; }
   // FP32 from 400000 cells on: 32 x 16 x 8, where a cell's share of the ring
   // shrinks further (mixed 80^3 0.972 against 0.945 ms, 96^3 1.020 against
   // 0.977, 128^3 1.39 against 1.32, 256^3, on its 128^3 level, 3.12 against
   // 3.03; also on 64^3 levels 128^3 takes 1.37).  64 x 8 x 8 and 32 x 16 x 16
   // are slower (128^3 1.31 and 1.53 when this one took 1.29), and in FP64 no
   // other shape gains.
-  static bool tall_block(long cells) { return sizeof(T) == 4 && cells > 400000L; }
+  static constexpr long TALL_BLOCK = 400000;
+  static bool tall_block(long cells) { return sizeof(T) == 4 && cells > TALL_BLOCK; }
   // The prolongation in the launch works on the whole ring: it pays up to
   // 200000 cells (96^3 FP64 2.11 ms with it on the fine level, 2.00 without;
   // mixed 128^3 1.45 and 1.36).
-  static bool prolong_in_block(long cells) { return cells <= 200000L; }
+  static constexpr long PROLONG_BLOCK = 200000;
+  static bool prolong_in_block(long cells) { return cells <= PROLONG_BLOCK; }
+  // whether blocks of this shape start from PRE on some level
+  static constexpr bool block_shape(BlockSmall, int) { return true; }
+  static constexpr bool block_shape(BlockLarge, int pre) { return pre != SW_PROLONG || LARGE_BLOCK < PROLONG_BLOCK; }
+  static constexpr bool block_shape(BlockTall, int pre) {
+    return sizeof(T) == 4 && (pre != SW_PROLONG || TALL_BLOCK < PROLONG_BLOCK);
+  }
 
   // arguments of a k_block launch (x -> x2) with blocks B, and their number;
   // c as for sweep_args
@@ -465,14 +475,13 @@ struct Ops {
   // to_caller as for sweep).  NORM (FP64, from x): the blocks' partial sums of
   // |b - A x_in|^2 go to partial; returns their number.
   template <typename B, int NIT, int PRE, bool NORM = false, bool REST = false>
-  int block_launch(DevLevel<T>& d, const DevLevel<T>* c, T omega, bool to_caller, double* partial, T* out) {
+  int block_launch(DevLevel<T>& d, const DevLevel<T>* c, T omega, bool to_caller, double* partial) {
     using S = BlockShape<T, B, NIT, PRE, REST>;
     BlockArgs<T> A = block_args<B>(d, c, omega);
     if (REST) {
       A.bc = c->b;
       A.RW = d.RW();
     }
-    if (out) A.xo = out;
     if (to_caller) {
       A.ext = caller_sol;
       A.U = caller_lvl;
@@ -486,16 +495,16 @@ struct Ops {
     hipLaunchKernelGGL((k_block<T, B, NIT, PRE, NORM, REST>), dim3((unsigned)nb), dim3(B::NT), S::LDS * sizeof(T), s, A);
     timer_end(timed, NIT);
     d.fused_up = true;
-    if (!out) std::swap(d.x, d.x2);
+    std::swap(d.x, d.x2);
     return nb;
   }
   template <int NIT, int PRE, bool NORM = false>
-  int block(DevLevel<T>& d, const DevLevel<T>* c, T omega, bool to_caller = false, double* partial = nullptr,
-            T* out = nullptr) {
-    if constexpr (sizeof(T) == 4 && PRE != SW_PROLONG && !NORM)
-      if (tall_block(d.cells())) return block_launch<BlockTall, NIT, PRE, NORM>(d, c, omega, to_caller, partial, out);
-    return large_block(d.cells()) ? block_launch<BlockLarge, NIT, PRE, NORM>(d, c, omega, to_caller, partial, out)
-                          : block_launch<BlockSmall, NIT, PRE, NORM>(d, c, omega, to_caller, partial, out);
+  int block(DevLevel<T>& d, const DevLevel<T>* c, T omega, bool to_caller = false, double* partial = nullptr) {
+    if constexpr (block_shape(BlockTall(), PRE) && !NORM)
+      if (tall_block(d.cells())) return block_launch<BlockTall, NIT, PRE, NORM>(d, c, omega, to_caller, partial);
+    if constexpr (block_shape(BlockLarge(), PRE))
+      if (large_block(d.cells())) return block_launch<BlockLarge, NIT, PRE, NORM>(d, c, omega, to_caller, partial);
+    return block_launch<BlockSmall, NIT, PRE, NORM>(d, c, omega, to_caller, partial);
   }
 
   // the same, then the residual restricted into c's b
@@ -503,11 +512,11 @@ struct Ops {
   void block_restrict(DevLevel<T>& d, const DevLevel<T>* c, T omega) {
     if constexpr (sizeof(T) == 4) {
       if (large_block(d.cells())) {
-        block_launch<BlockLarge, NIT, PRE, false, true>(d, c, omega, false, nullptr, nullptr);
+        block_launch<BlockLarge, NIT, PRE, false, true>(d, c, omega, false, nullptr);
         return;
       }
     }
-    block_launch<BlockSmall, NIT, PRE, false, true>(d, c, omega, false, nullptr, nullptr);
+    block_launch<BlockSmall, NIT, PRE, false, true>(d, c, omega, false, nullptr);
   }
   // The residual needs a ring one cell wider (two along x), so joining the
   // restriction pays on smaller levels than the iterations do: up to 150000

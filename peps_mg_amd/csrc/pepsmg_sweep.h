@@ -1,4 +1,4 @@
-// pepsmg_sweep.h -- NIT red/black iterations in one pass over a level
+// pepsmg_sweep.h -- NIT = 2 red/black iterations in one pass over a level
 // (gfx950), from x, from x = 0 (src/multigrid.f90:1937) or from x plus the
 // prolongation of the coarser level (:1958-1959 with :1676-1754), out of
 // place.
@@ -122,6 +122,7 @@ struct SweepShape {
   static constexpr int RING = 2 * NIT;
   // SW_PROLONG: the outermost pair only feeds the interpolation of the next
   static constexpr int RINGX = RING + (PRE == SW_PROLONG ? 2 : 0);
+  static_assert(NIT == 2, "the march runs four half-sweeps in groups of six plane steps");
   static constexpr int NS = 2 * NIT + 2;            // planes in registers
   static constexpr int NBR = 2 * NIT - 2, NBB = 2 * NIT - 1;   // red / black half planes of b waiting in LDS
   static constexpr int EDGE = 2 * (WAVES + 1) * 64;      // one kind of edge rows of one plane
@@ -491,10 +492,8 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
     };
     half(std::integral_constant<int, 1>());
     half(std::integral_constant<int, 2>());
-    if constexpr (NIT > 1) {
-      half(std::integral_constant<int, 3>());
-      half(std::integral_constant<int, 4>());
-    }
+    half(std::integral_constant<int, 3>());
+    half(std::integral_constant<int, 4>());
     // ---- b of plane m - 1 into its slots, black cells of plane m to the neighbours ----
     {
       constexpr int KP = ODD ? 0 : 1;                // parity of plane m - 1
@@ -503,7 +502,7 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
       for (int r = 0; r < R; r++) {
         const bool rf = ((r + 1 + KP) & 1) == 0;     // red is the first cell
         bblk[(sb * R + r) * NT + ct] = rf ? bc[r].y : bc[r].x;
-        if (NIT > 1) bred[((U & 1) * R + r) * NT + ct] = rf ? bc[r].x : bc[r].y;
+        bred[((U & 1) * R + r) * NT + ct] = rf ? bc[r].x : bc[r].y;
       }
       if (PRE != SW_ZERO) {
         constexpr int KM = ODD ? 1 : 0;              // parity of plane m
@@ -521,10 +520,8 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
       step(m + 1, std::integral_constant<int, 1>(), std::true_type());
       step(m + 2, std::integral_constant<int, 2>(), std::true_type());
       step(m + 3, std::integral_constant<int, 3>(), std::true_type());
-      if constexpr (NS > 4) {
-        step(m + 4, std::integral_constant<int, 4>(), std::true_type());
-        step(m + 5, std::integral_constant<int, 5>(), std::true_type());
-      }
+      step(m + 4, std::integral_constant<int, 4>(), std::true_type());
+      step(m + 5, std::integral_constant<int, 5>(), std::true_type());
       m += NS;
     }
     auto run = [&](auto Uc) {
@@ -535,10 +532,8 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
     run(std::integral_constant<int, 1>());
     run(std::integral_constant<int, 2>());
     run(std::integral_constant<int, 3>());
-    if constexpr (NS > 4) {
-      run(std::integral_constant<int, 4>());
-      run(std::integral_constant<int, 5>());
-    }
+    run(std::integral_constant<int, 4>());
+    run(std::integral_constant<int, 5>());
     m += NS;
   }
 }
