@@ -411,15 +411,31 @@ struct Ops {
     std::swap(d.x, d.x2);
   }
 
-  // Whether iterations on level d run by blocks of the level in LDS (k_block):
-  // up to 1.2 M cells in FP64 and 3 M in FP32, where the launches they save
-  // outweigh the rings.  Solves against one launch per iteration: FP64 16^3
-  // 0.80 against 0.93 ms, 64^3 1.57 against 1.76, 96^3 2.14 against 2.44 (by
-  // blocks on its 128^3 level, 128^3 takes 2.99 against 2.81); mixed 32^3 0.59
-  // against 0.70 ms, 64^3 0.80 against 0.99, 96^3 1.05 against 1.31, 128^3
-  // 1.47 against 1.54.
+  // Whether iterations on level d run by blocks of the level in LDS (k_block),
+  // where the launches they save outweigh the rings.  Solves against one
+  // launch per iteration: FP64 16^3 0.80 against 0.93 ms, 64^3 1.20 against
+  // 1.24, 96 x 64 x 80 1.51 against 1.59; mixed 32^3 0.59 against 0.70 ms,
+  // 64^3 0.73 against 0.81, 96^3 0.95 against 1.05, 144 x 128 x 128 1.84
+  // against 1.98, 144 x 144 x 128 2.02 against 2.03.
+  // FP32: up to 3 M cells.  (From there to the sweeps' 4 M one launch per
+  // iteration: 160 x 144 x 144 2.37 against 2.50 ms by blocks; sweeps would
+  // take 2.17, and 144^3, 2.28 by blocks, 2.02.)
+  // FP64: while the large blocks, one to a CU, all run at once.  A second
+  // wave of them costs what single iterations do and more: 64 x 64 x 128 (256
+  // blocks) 1.49 against 1.55 ms, 80^3 (300) 1.74 against 1.68, 128 x 64 x 96
+  // (384) 1.55 against 1.42, 64 x 128 x 128 (512) 1.63 against 1.56, 112 x 96
+  // x 96 (576) 2.47 against 2.32.  Only where that wave is four fifths full
+  // and the rows fill three quarters of the single iterations' tiles or less
+  // do blocks gain: 96^3 (432) 1.63 against 1.66, 96 x 96 x 112 (504) 2.14
+  // against 2.19, but 96 x 96 x 80 (360) 1.88 against 1.83.
+  // A batch's launch takes its items' blocks together: there by their cells.
   static bool blocks(long cells) { return cells <= (sizeof(T) == 8 ? 1200000L : 3000000L); }
-  bool blocks(const DevLevel<T>& d) const { return !single() && blocks(d.cells()); }
+  bool blocks(const DevLevel<T>& d) const {
+    if (single()) return false;
+    if (sizeof(T) == 4 || d.cells() <= LARGE_BLOCK) return blocks(d.cells());
+    const long n = block_count<BlockLarge>(d), cus = cu_count();
+    return n <= cus || (n <= 2 * cus && 5 * n >= 4 * 2 * cus && 4L * d.nx <= 3L * ((d.nx + FTX - 1) / FTX) * FTX);
+  }
   // 32 x 8 x 8 blocks of 1024 threads from 300000 cells on in FP64 and 150000
   // in FP32: less ring per cell (96^3 FP64 2.14 against 2.38 ms); below,
   // 16 x 8 x 4 keeps more CUs busy (64^3 FP64 1.56 against 1.69 ms when its

@@ -23,7 +23,10 @@ def sdm_from(g):
 # partial tiles along x and y, odd plane counts (the top chunk ends on an even plane and the downward march starts one
 # plane above the domain), odd rows; stretched where the axis is even
 FP64 = [((70, 520, 37), (1.01, 1.003, 1.0), "64, 32"), ((130, 150, 71), (1.01, 1.01, 1.0), "64, 8"),
-        ((171, 157, 51), (1.0, 1.0, 1.0), "64, 8"), ((128, 128, 128), (1.0, 1.0, 1.01), "64, 32")]
+        ((171, 157, 51), (1.0, 1.0, 1.0), "64, 8"), ((128, 128, 128), (1.0, 1.0, 1.01), "64, 32"),
+        # more large blocks than CUs: 300, 405 and 576
+        ((80, 80, 80), (1.01, 1.0, 1.0), "64, 8"), ((131, 67, 69), (1.0, 1.0, 1.0), "64, 8"),
+        ((96, 96, 128), (1.0, 1.01, 1.0), "64, 8")]
 
 
 @pytest.mark.parametrize("dims,stretch,tile", FP64)

@@ -24,7 +24,7 @@ def bench_name(mg, precision):
 
 @pytest.mark.parametrize("n,precision,symbol", [
     (32, 0, "k_block<double, pepsmg::BlockTile<16, 8, 4, 512>, 2, 0, false, false>"),
-    (80, 0, "k_block<double, pepsmg::BlockTile<32, 8, 8, 1024>, 2, 0, false, false>"),
+    (72, 0, "k_block<double, pepsmg::BlockTile<32, 8, 8, 1024>, 2, 0, false, false>"),
     (48, 1, "k_block<float, pepsmg::BlockTile<16, 8, 4, 512>, 2, 0, false, false>"),
     (64, 1, "k_block<float, pepsmg::BlockTile<32, 8, 8, 1024>, 2, 0, false, false>"),
     (80, 1, "k_block<float, pepsmg::BlockTile<32, 16, 8, 1024>, 2, 0, false, false>")])
