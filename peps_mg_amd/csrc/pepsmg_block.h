@@ -10,13 +10,12 @@
 // tile and a ring of 2 NIT cells in LDS: all loads are issued at the start
 // (one round trip), the half-sweeps follow with a barrier each, every one on
 // a region one cell smaller, and the tile is stored.  Levels this small are
-// served from the caches, so the ring (7.5 times the tile's cells for 16 x 8
+// served from the caches, so the ring (8 times the tile's cells for 16 x 8
 // x 4 and two iterations) costs little beside the launches it saves.
 //
 // Threads own pairs (i odd, i + 1) of the region through the whole launch;
 // LDS keeps the first and the second cells of the pairs apart, so lanes touch
-// consecutive words.  Values, expressions and operand order are those of the
-// separate kernels (FP64 bit for bit).
+// consecutive words.  Values are those of the separate kernels bit for bit.
 #pragma once
 #include "pepsmg_coarse.h"
 #include "pepsmg_sweep.h"

@@ -357,9 +357,15 @@ struct Ops {
   // the chunks mostly ring).  Solves, both ways:
   // FP64 128^3 (share 0.11) 3.29 against 3.13 ms, 160^3 (0.16) 4.99 against
   // 5.10, 192^3 5.08 against 5.35, 320^3 13.5 against 15.4, 512^3 39.1
-  // against 42.8; mixed 128^3 (0.11) 1.55 against 1.57, 160^3 1.97 against 2.21, 256^3 3.22 against 3.78, 384^3 6.49
-  // against 9.89, 512^3 13.1 against 17.5.  (A plane's row offsets are
-  // 32-bit bytes.)
+  // against 42.8; mixed 128^3 (0.11) 1.55 against 1.57, 160^3 1.97 against
+  // 2.21, 256^3 3.22 against 3.78, 384^3 6.49 against 9.89, 512^3 13.1 against
+  // 17.5.  Between 2.5 M and 4 M cells mixed solves would gain (160 x 160 x
+  // 128 1.39 against 1.59 ms), FP64 ones a little (2.77 against 2.85).
+  // With z stretched no plane has kept divisors (zlo, zhi): a launch takes
+  // 0.99 ms in FP64 and 0.55 in FP32 at 512^3, against 1.1 and 0.55 for the
+  // two it replaces; solves before and after the sweeps FP64 256^3 7.72 and
+  // 7.22, 320^3 16.7 and 13.4, 512^3 42.9 and 41.3; mixed 256^3 3.63 and 3.26,
+  // 512^3 17.6 and 16.7.  (A plane's row offsets are 32-bit bytes.)
   bool sweeps(const DevLevel<T>& d) const {
     if (single() || d.cells() < 4000000L || d.pxy * (long)sizeof(T) > 0x7fffffffL) return false;
     double share = 0.0;
