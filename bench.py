@@ -273,20 +273,24 @@ def workload_rhs_device(n, lz, sdm, torch):
 
 
 def vcycle_roofline(n, levels, t, cycles):
-    """Whole FP64 V(2,2) cycle against the HBM peak: algorithmic elements per
-    cycle E = n (16.25 sum_{l<L} 8^-l + 2) (per level four red/black
-    iterations at 3 n, residual + restriction and prolongation + correction
-    at 2.125 n each; the convergence residual at 2 n on the finest level),
-    8 bytes each, over the measured time per cycle."""
+    """Whole FP64 V(2,2) cycle as a rate of work: the elements a cycle would
+    move with one pass per operation, E = n (16.25 sum_{l<L} 8^-l + 2) (per
+    level four red/black iterations at 3 n, residual + restriction and
+    prolongation + correction at 2.125 n each; the convergence residual at
+    2 n on the finest level), 8 bytes each, over the measured time per cycle
+    and against the HBM peak.  Not a bandwidth: large levels take two
+    iterations in one pass."""
     e = n ** 3 * (16.25 * sum(8.0 ** -l for l in range(levels)) + 2.0)
     ms = t / cycles * 1e3
     gbs = e * 8 / (ms * 1e-3) / 1e9
     return {"bytes_per_cycle": round(e * 8), "ms_per_cycle": round(ms, 4), "achieved_gbs": round(gbs, 1),
             "frac": round(gbs / HBM_PEAK_GBS, 4),
-            "model": "4 red/black iterations (3 n each), residual+restriction and prolongation+correction "
-                     "(2.125 n each) per level, the convergence residual (2 n) once; the solver folds that "
-                     "residual into the next cycle's first smoothing pass and reads no x in the first "
-                     "iteration on coarse levels, so it moves fewer bytes than counted"}
+            "model": "a rate of work, not a bandwidth: 4 red/black iterations (3 n each), residual+restriction and "
+                     "prolongation+correction (2.125 n each) per level and the convergence residual (2 n) once, "
+                     "each counted as a pass of its own; the solver takes two iterations in one pass where that "
+                     "is faster (512^3: the post-smoothing; its coarse levels: both legs), folds that residual "
+                     "into the next cycle's first smoothing pass and reads no x in the first iteration on "
+                     "coarse levels, so it moves fewer bytes than counted"}
 
 
 def iterations_per_launch(kernel):

@@ -373,16 +373,17 @@ static __global__ void __launch_bounds__(RED_THREADS) k_dot_final(const double* 
 // A scalar of the CG smoother as the partial sums it consists of: every block
 // of the kernel that needs it adds them up itself, in k_dot_final's order (so
 // all get k_dot_final's value), instead of waiting for a launch of one block
-// in between.  n = 1: the scalar itself.
+// in between.  FOLD = false: p points to the scalar itself.
 struct PartialSum {
   const double* p;
   int n;
 };
 // The quotient num / den of two such scalars on every thread; both sums are
 // formed side by side (sh: 2 RED_THREADS / 64 doubles).
+template <bool FOLD>
 __device__ __forceinline__ double partial_ratio(const PartialSum& num, const PartialSum& den, double* sh) {
   constexpr int NW = RED_THREADS / 64;
-  if (num.n == 1 && den.n == 1) return num.p[0] / den.p[0];
+  if (!FOLD) return num.p[0] / den.p[0];
   double a = 0.0, d = 0.0;
   const int n = max(num.n, den.n);
   for (int c = threadIdx.x; c < n; c += RED_THREADS) {

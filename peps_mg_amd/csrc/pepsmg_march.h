@@ -325,13 +325,13 @@ k_refine_step(const double* __restrict__ x, const float* __restrict__ e, const d
 // formed while staging, stored for the tile cells, Ap = A pnew stored in
 // ap, partial sums of (Ap, pnew) (:206-207).  p and pnew are different
 // arrays (neighbouring tiles still read p).
-template <typename T, int TY>
+template <typename T, int TY, bool FOLD>
 __global__ void __launch_bounds__(MARCH_THREADS)
 k_cg_ap_fold(const T* __restrict__ r, const T* __restrict__ p, T* __restrict__ pnew, T* __restrict__ ap, Lvl<T> L,
              MarchGrid G, double* __restrict__ partial, PartialSum rnew, PartialSum rold) {
   static_assert(MARCH_THREADS == RED_THREADS, "partial_ratio's order");
   __shared__ double shs[2 * MARCH_THREADS / 64];
-  const T beta = (T)partial_ratio(rnew, rold, shs);
+  const T beta = (T)partial_ratio<FOLD>(rnew, rold, shs);
   resid_march_block<T, TY, 7>(blockIdx.x, r, (const float*)nullptr, p, ap, (float*)nullptr, pnew, L, G, partial, L, L,
                               (T*)nullptr, L, beta);
 }

@@ -87,13 +87,13 @@ k_cg_start0(T* __restrict__ r, T* __restrict__ p, const T* __restrict__ b, Lvl<T
 }
 
 // x = x + alpha p, r = r - alpha Ap (:209-216), partial (r, r) (:221)
-template <typename T>
+template <typename T, bool FOLD>
 __global__ void __launch_bounds__(64 * CG_WAVES)
 k_cg_xr(T* __restrict__ x, T* __restrict__ r, const T* __restrict__ p, const T* __restrict__ ap,
         PartialSum rr, PartialSum pap, Lvl<T> L, bool zero_x, double* __restrict__ partial) {
   static_assert(64 * CG_WAVES == RED_THREADS, "partial_ratio's order");
   __shared__ double sh[2 * CG_WAVES];
-  const T alpha = (T)partial_ratio(rr, pap, sh);
+  const T alpha = (T)partial_ratio<FOLD>(rr, pap, sh);
   double acc = cg_rows(L, [&](long q, bool two) {
     if (two) {
       const auto pv = ld_pair(p + q), av = ld_pair(ap + q), rv = ld_pair(r + q);
@@ -305,8 +305,8 @@ static void cg_iterate(Ops<T>& op, DevLevel<T>& d, T* x, const T* b, T* r, T* p,
   for (int it = 0; it < nu; it++) {
     const int cur = it & 1, nxt = (it + 1) & 1;
     if (march && it > 0) {   // p = r + beta p (:223-229) folded into A p (:206-207)
-      hipLaunchKernelGGL((k_cg_ap_fold<T, RESID_TY>), dim3(mb), dim3(MARCH_THREADS), 0, op.s, r, p, p2, ap, d.L(),
-                         G, pap, rr[cur], rr[nxt]);
+      auto* k = fold ? k_cg_ap_fold<T, RESID_TY, true> : k_cg_ap_fold<T, RESID_TY, false>;
+      hipLaunchKernelGGL(k, dim3(mb), dim3(MARCH_THREADS), 0, op.s, r, p, p2, ap, d.L(), G, pap, rr[cur], rr[nxt]);
       ap2 = sum(pap, mb, 2);
       std::swap(p, p2);
     } else if (march) {                                             // :206-207
@@ -318,7 +318,8 @@ static void cg_iterate(Ops<T>& op, DevLevel<T>& d, T* x, const T* b, T* r, T* p,
       op.dot(d, ap, p, partial, sc + 2);
       ap2 = {sc + 2, 1};
     }
-    hipLaunchKernelGGL((k_cg_xr<T>), dim3(eb), eblk, 0, op.s, x, r, p, ap, rr[cur], ap2, d.L(), zero_x && it == 0,
+    auto* k = fold ? k_cg_xr<T, true> : k_cg_xr<T, false>;
+    hipLaunchKernelGGL(k, dim3(eb), eblk, 0, op.s, x, r, p, ap, rr[cur], ap2, d.L(), zero_x && it == 0,
                        prr[nxt]);                                   // partial (r, r) (:221)
     rr[nxt] = sum(prr[nxt], eb, nxt);
     if (!march && it + 1 < nu)
@@ -1468,7 +1469,7 @@ int pepsmg_cg_solver(const pepsmg_grid* grid, double* sol, const double* coeff, 
     const int cur = it & 1, nxt = (it + 1) & 1;
     op.apply(o.d, ap, p);                                          // :108
     op.dot(o.d, ap, p, o.partial, sc + 2);                         // :109
-    hipLaunchKernelGGL((k_cg_xr<double>), dim3(eb), eblk, 0, o.s, o.d.x, o.d.r, p, ap, PartialSum{sc + cur, 1},
+    hipLaunchKernelGGL((k_cg_xr<double, false>), dim3(eb), eblk, 0, o.s, o.d.x, o.d.r, p, ap, PartialSum{sc + cur, 1},
                        PartialSum{sc + 2, 1}, o.d.L(), false, o.partial);                                 // :111-118
     hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(RED_THREADS), 0, o.s, o.partial, eb, sc + nxt);   // :123
     rc = o.scalar(nxt, &t2);
