@@ -82,6 +82,12 @@ __device__ __forceinline__ double sw_shift(double v) {
 }
 __device__ __forceinline__ float sw_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double sw_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+// a f, rounded like the ordinary product, but 0 for f = 0 whatever a is
+__device__ __forceinline__ float sw_mul0(float a, float f) {
+  float r;
+  asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(f));
+  return r;
+}
 template <typename T>
 __device__ __forceinline__ T sw_west(T v) { return sw_shift<0x138>(v); }   // wave_shr:1
 template <typename T>
@@ -189,9 +195,8 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
   }
   // Planes zlo .. zhi share their z coefficients: there the divisors are
   // kept.  FP64: c0 and 1 / c0; FP32: omega / c0 alone.  Cells outside the
-  // level get the factor 0, which leaves them 0; FP32 also selects by lev
-  // (beside an infinity or a NaN the product with 0 is a NaN).
-  bool lev[R][2];
+  // level get the factor 0, which leaves them 0 (in FP32 also beside an
+  // infinity or a NaN: sw_mul0).
   T dv[F64 ? R : 1][2], rv[R][2];
   bool kept = A.zhi >= A.zlo;
 #pragma unroll
@@ -199,7 +204,6 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
 #pragma unroll
     for (int c = 0; c < 2; c++) {
       const bool in = (c ? in1 : in0) && j0 + r <= L.ny;
-      lev[r][c] = in;
       const T c0 = -(c1[c] + c2[c] + c3[r] + c4[r] + A.c5u + A.c6u);
       if constexpr (F64) {
         dv[r][c] = c0;
@@ -468,10 +472,7 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs<T>& A, int lin) {
           for (int r = 0; r < R; r++) put(r, q[r]);
         } else if constexpr (FAST) {
 #pragma unroll
-          for (int r = 0; r < R; r++) {
-            const T q = diff(r, A.c5u, A.c6u) * rv[r][cell(r)];
-            put(r, lev[r][cell(r)] ? q : T(0));
-          }
+          for (int r = 0; r < R; r++) put(r, sw_mul0(diff(r, A.c5u, A.c6u), rv[r][cell(r)]));
         } else {
           const T c5 = ldc(L.cwz, k), c6 = ldc(L.cez, k);
 #pragma unroll
