@@ -28,7 +28,7 @@
 // 512^3, two iterations: 4 rows x 8 waves 400 us, 8 x 8 387 us but the
 // variant with the prolongation spills, 4 x 12 404 us).
 // At 512^3, two iterations: FP64 0.85 ms against 2 x 0.55 ms for k_rb_fused;
-// FP32 from x 0.40 against 2 x 0.28, from 0 0.26 against 0.49, with the
+// FP32 from x 0.38 against 2 x 0.28, from 0 0.26 against 0.49, with the
 // prolongation 0.42 against 0.75 ms for its three launches.  FP32 reads
 // 1.10x and writes 1.00x the bytes of one pass.  FP64 is held back by its
 // arithmetic (about 500 vector operations a wave and step), FP32 by the
