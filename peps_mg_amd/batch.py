@@ -52,7 +52,8 @@ class BatchSolver:
 
     def set_tiles(self, tile_x=None, tile_y=None):
         """Fused-smoother tile shape per problem (lists of nprob; None or 0:
-        the options' values)."""
+        the options' values).  Problems with a tile run one iteration a
+        launch."""
         n = len(self.sdms)
         ax = (C.c_int32 * n)(*tile_x) if tile_x is not None else None
         ay = (C.c_int32 * n)(*tile_y) if tile_y is not None else None
